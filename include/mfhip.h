@@ -467,6 +467,14 @@ MFH_API int mfh_plane_mean_backward(uint64_t dy, uint64_t dx, int64_t planes, in
  * Replaces MSELoss.forward, ops/loss.py:99-106. */
 MFH_API int mfh_mse_loss(uint64_t pred, uint64_t target, uint64_t loss, int64_t count, uint64_t stream);
 
+/* Doubles of workspace with which mfh_mse_loss_split forms the loss of count elements on several
+ * workgroups (0: one workgroup is enough, use mfh_mse_loss; -1: count out of range). */
+MFH_API int64_t mfh_mse_loss_workspace(int64_t count);
+
+/* mfh_mse_loss over several workgroups, whose FP64 sums (in `workspace`) a second launch adds. */
+MFH_API int mfh_mse_loss_split(uint64_t pred, uint64_t target, uint64_t loss, int64_t count, uint64_t workspace,
+                               int64_t workspace_doubles, uint64_t stream);
+
 /* grad = seed[0] * ((2 * (pred - target)) / float(count)), each operation rounded to float32, or
  * grad += that when add != 0 (seed: the loss gradient, one float on the device).
  * Replaces MSELoss.backward, ops/loss.py:108-113. */

@@ -1081,7 +1081,23 @@ MFH_API int mfh_mse_loss(std::uint64_t pred, std::uint64_t target, std::uint64_t
     MFH_REQUIRE(count >= 0 && fits_index(count), "mse element count out of range");
     MFH_REQUIRE(loss && (count == 0 || (pred && target)), "mse loss received a null buffer");
     return launch_mse_loss(as_ptr<const float>(pred), as_ptr<const float>(target), as_ptr<float>(loss), count,
-                           as_stream(stream));
+                           nullptr, as_stream(stream));
+}
+
+MFH_API std::int64_t mfh_mse_loss_workspace(std::int64_t count) {
+    if (count < 0 || !fits_index(count)) return -1;
+    const int groups = mse_loss_groups(count);
+    return groups > 1 ? groups : 0;
+}
+
+MFH_API int mfh_mse_loss_split(std::uint64_t pred, std::uint64_t target, std::uint64_t loss, std::int64_t count,
+                               std::uint64_t workspace, std::int64_t workspace_doubles, std::uint64_t stream) {
+    MFH_TRY(require_ready());
+    MFH_REQUIRE(count >= 0 && fits_index(count), "mse element count out of range");
+    MFH_REQUIRE(loss && (count == 0 || (pred && target)), "mse loss received a null buffer");
+    MFH_REQUIRE(workspace && workspace_doubles >= mse_loss_groups(count), "mse loss workspace too small");
+    return launch_mse_loss(as_ptr<const float>(pred), as_ptr<const float>(target), as_ptr<float>(loss), count,
+                           as_ptr<double>(workspace), as_stream(stream));
 }
 
 MFH_API int mfh_mse_loss_backward(std::uint64_t pred, std::uint64_t target, std::uint64_t seed, std::uint64_t grad,

@@ -7,7 +7,9 @@
 //   * loss = float(FP64 sum of float32 (d * d) / count), d = pred - target (float32 difference and
 //     square, as the operator's diff * diff)
 //   * its gradient g[i] (+)= seed * ((2 * d) / float(count))             (float32, in that order)
-//   * column sums out[j] = float(FP64 sum over rows of src[r, j]), rows in order.
+//   * column sums out[j] = float(FP64 sum over rows of src[r, j]), 16 runs of rows, each in order, then in
+//     run order.
+#include <algorithm>
 #include <cstdint>
 
 #include "common.h"
@@ -18,14 +20,30 @@ namespace {
 constexpr int HEAD_THREADS = 256;
 constexpr int LOSS_THREADS = 1024;  // one workgroup forms the loss
 
+// LANES lanes share a plane: lane l adds elements l, l + LANES, ... in FP64 (four loads in flight),
+// then a fixed butterfly adds the lanes. One thread per plane read a cache line per lane and element
+// and left all but planes / 64 waves idle: 64 x 64 planes of 29 x 39 took 324 us for 18.5 MB
+// (the stem's whole training pass went from 677 to 336 us with the lanes below).
+template <int LANES>
 __global__ __launch_bounds__(HEAD_THREADS) void plane_mean_kernel(const float* __restrict__ x, float* __restrict__ y,
                                                                   long long planes, int hw) {
-    const long long p = static_cast<long long>(blockIdx.x) * HEAD_THREADS + threadIdx.x;
-    if (p >= planes) return;
+    const long long p = (static_cast<long long>(blockIdx.x) * HEAD_THREADS + threadIdx.x) / LANES;
+    if (p >= planes) return;  // uniform over the LANES lanes of a plane
+    const int lane = threadIdx.x % LANES;
     const float* __restrict__ src = x + p * hw;
     double s = 0.0;
-    for (int i = 0; i < hw; ++i) s += static_cast<double>(src[i]);
-    y[p] = static_cast<float>(s / static_cast<double>(hw));
+    int i = lane;
+    for (; i + 3 * LANES < hw; i += 4 * LANES) {
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = src[i + u * LANES];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s += static_cast<double>(v[u]);
+    }
+    for (; i < hw; i += LANES) s += static_cast<double>(src[i]);
+#pragma unroll
+    for (int offset = LANES / 2; offset > 0; offset >>= 1) s += __shfl_xor(s, offset, LANES);
+    if (lane == 0) y[p] = static_cast<float>(s / static_cast<double>(hw));
 }
 
 __global__ __launch_bounds__(HEAD_THREADS) void plane_mean_backward_kernel(const float* __restrict__ dy, float* dx,
@@ -37,28 +55,68 @@ __global__ __launch_bounds__(HEAD_THREADS) void plane_mean_backward_kernel(const
     dx[i] = add ? dx[i] + v : v;
 }
 
-// One workgroup: thread t adds the squares of elements t, t + LOSS_THREADS, ... in FP64; the
-// thread sums are then combined by a fixed tree in LDS.
-__global__ __launch_bounds__(LOSS_THREADS) void mse_loss_kernel(const float* __restrict__ pred,
-                                                                const float* __restrict__ target,
-                                                                float* __restrict__ loss, long long count) {
-#pragma clang fp contract(off)
-    __shared__ double partial[LOSS_THREADS];
-    double s = 0.0;
-    for (long long i = threadIdx.x; i < count; i += LOSS_THREADS) {
-        const float d = pred[i] - target[i];
-        const float square = d * d;
-        s += static_cast<double>(square);
-    }
+// The squared differences of 256 x 1000 outputs took one workgroup 70 us, a load at a time; a CU's own
+// bandwidth bounds it, so larger counts take several workgroups. The sums are formed by LOSS_THREADS-thread workgroups: thread t of the grid adds
+// those of elements t, t + threads, ... in that order in FP64 with LOSS_AHEAD loads of each operand
+// in flight; a workgroup's thread sums are combined by a fixed tree in LDS. A single workgroup
+// writes the loss; several write their sums to partials, which mse_finish_kernel adds.
+constexpr int LOSS_AHEAD = 8;
+
+__device__ __forceinline__ double tree_sum(double* partial, double s) {
     partial[threadIdx.x] = s;
     __syncthreads();
     for (int half = LOSS_THREADS / 2; half > 0; half >>= 1) {
         if (static_cast<int>(threadIdx.x) < half) partial[threadIdx.x] += partial[threadIdx.x + half];
         __syncthreads();
     }
-    // The mean of no elements is NaN, as the operator's FP64 mean of an empty array.
-    if (threadIdx.x == 0)
-        loss[0] = count > 0 ? static_cast<float>(partial[0] / static_cast<double>(count)) : __builtin_nanf("");
+    return partial[0];
+}
+
+// The mean of no elements is NaN, as the operator's FP64 mean of an empty array.
+__device__ __forceinline__ float mean_of(double sum, long long count) {
+    return count > 0 ? static_cast<float>(sum / static_cast<double>(count)) : __builtin_nanf("");
+}
+
+__global__ __launch_bounds__(LOSS_THREADS) void mse_loss_kernel(const float* __restrict__ pred,
+                                                                const float* __restrict__ target,
+                                                                float* __restrict__ loss,
+                                                                double* __restrict__ partials, long long count) {
+#pragma clang fp contract(off)
+    __shared__ double partial[LOSS_THREADS];
+    const long long step = static_cast<long long>(gridDim.x) * LOSS_THREADS;
+    long long i = static_cast<long long>(blockIdx.x) * LOSS_THREADS + threadIdx.x;
+    double s = 0.0;
+    for (; i + (LOSS_AHEAD - 1) * step < count; i += LOSS_AHEAD * step) {
+        float p[LOSS_AHEAD], t[LOSS_AHEAD];
+#pragma unroll
+        for (int u = 0; u < LOSS_AHEAD; ++u) {
+            p[u] = pred[i + u * step];
+            t[u] = target[i + u * step];
+        }
+#pragma unroll
+        for (int u = 0; u < LOSS_AHEAD; ++u) {
+            const float d = p[u] - t[u];
+            const float square = d * d;
+            s += static_cast<double>(square);
+        }
+    }
+    for (; i < count; i += step) {
+        const float d = pred[i] - target[i];
+        const float square = d * d;
+        s += static_cast<double>(square);
+    }
+    const double sum = tree_sum(partial, s);
+    if (threadIdx.x != 0) return;
+    if (partials) partials[blockIdx.x] = sum;
+    else loss[0] = mean_of(sum, count);
+}
+
+// The workgroups' sums (at most LOSS_THREADS), added by the same tree.
+__global__ __launch_bounds__(LOSS_THREADS) void mse_finish_kernel(const double* __restrict__ partials, int groups,
+                                                                  float* __restrict__ loss, long long count) {
+    __shared__ double partial[LOSS_THREADS];
+    const double sum = tree_sum(partial, static_cast<int>(threadIdx.x) < groups ? partials[threadIdx.x] : 0.0);
+    if (threadIdx.x == 0) loss[0] = mean_of(sum, count);
 }
 
 __global__ __launch_bounds__(HEAD_THREADS) void mse_grad_kernel(const float* __restrict__ pred,
@@ -73,21 +131,36 @@ __global__ __launch_bounds__(HEAD_THREADS) void mse_grad_kernel(const float* __r
     grad[i] = add ? grad[i] + v : v;
 }
 
-__global__ __launch_bounds__(HEAD_THREADS) void column_sums_kernel(const float* __restrict__ src,
-                                                                   float* __restrict__ out, long long rows,
-                                                                   long long cols) {
-    const long long j = static_cast<long long>(blockIdx.x) * HEAD_THREADS + threadIdx.x;
-    if (j >= cols) return;
+// A workgroup of COLUMN_SPAN columns by COLUMN_GROUPS row groups: group g adds its run of rows in
+// order in FP64, eight loads in flight; the groups' sums are then added in group order through LDS.
+// Latency bounds it: one thread per column walked 256 rows of 1000 columns in 12.6 us.
+constexpr int COLUMN_SPAN = 64, COLUMN_GROUPS = 16;
+
+__global__ __launch_bounds__(COLUMN_SPAN* COLUMN_GROUPS) void column_sums_kernel(const float* __restrict__ src,
+                                                                                 float* __restrict__ out,
+                                                                                 long long rows, long long cols) {
+    __shared__ double group_sum[COLUMN_GROUPS][COLUMN_SPAN];
+    const int c = threadIdx.x % COLUMN_SPAN, g = threadIdx.x / COLUMN_SPAN;
+    const long long j = static_cast<long long>(blockIdx.x) * COLUMN_SPAN + c;
+    const long long per = (rows + COLUMN_GROUPS - 1) / COLUMN_GROUPS;
+    const long long last = min(rows, (g + 1) * per);
     double s = 0.0;
-    long long r = 0;
-    for (; r + 8 <= rows; r += 8) {  // eight loads in flight, added in row order
-        float v[8];
+    if (j < cols) {
+        long long r = g * per;
+        for (; r + 8 <= last; r += 8) {
+            float v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = src[(r + u) * cols + j];
+            for (int u = 0; u < 8; ++u) v[u] = src[(r + u) * cols + j];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) s += static_cast<double>(v[u]);
+            for (int u = 0; u < 8; ++u) s += static_cast<double>(v[u]);
+        }
+        for (; r < last; ++r) s += static_cast<double>(src[r * cols + j]);
     }
-    for (; r < rows; ++r) s += static_cast<double>(src[r * cols + j]);
+    group_sum[g][c] = s;
+    __syncthreads();
+    if (g != 0 || j >= cols) return;
+#pragma unroll
+    for (int h = 1; h < COLUMN_GROUPS; ++h) s += group_sum[h][c];
     out[j] = static_cast<float>(s);
 }
 
@@ -95,7 +168,14 @@ __global__ __launch_bounds__(HEAD_THREADS) void column_sums_kernel(const float* 
 
 int launch_plane_mean(const float* x, float* y, std::int64_t planes, int hw, hipStream_t stream) {
     if (planes == 0) return OK;
-    launch(plane_mean_kernel, blocks_for(planes, HEAD_THREADS), HEAD_THREADS, 0, stream, x, y, planes, hw);
+    // A wave per plane from two full passes of it on; 16 lanes for the small planes of a network's end
+    // (4 x 5, 7 x 7), of which a wave then takes four; one thread where 16 lanes would mostly idle.
+    const auto run = [&](auto kernel, int lanes) {
+        launch(kernel, blocks_for(planes * lanes, HEAD_THREADS), HEAD_THREADS, 0, stream, x, y, planes, hw);
+    };
+    if (hw >= 128) run(plane_mean_kernel<64>, 64);
+    else if (hw >= 16) run(plane_mean_kernel<16>, 16);
+    else run(plane_mean_kernel<1>, 1);
     return MFH_CHECK_LAUNCH("plane_mean", stream);
 }
 
@@ -107,9 +187,22 @@ int launch_plane_mean_backward(const float* dy, float* dx, std::int64_t planes, 
     return MFH_CHECK_LAUNCH("plane_mean_backward", stream);
 }
 
-int launch_mse_loss(const float* pred, const float* target, float* loss, std::int64_t count, hipStream_t stream) {
-    launch(mse_loss_kernel, 1, LOSS_THREADS, 0, stream, pred, target, loss, count);
-    return MFH_CHECK_LAUNCH("mse_loss", stream);
+// Workgroups of the loss of count elements: one while its loads are a few rounds (a second launch
+// costs about 3 us), else one per LOSS_AHEAD rounds up to the device's CUs.
+int mse_loss_groups(std::int64_t count) {
+    if (count <= 4LL * LOSS_AHEAD * LOSS_THREADS) return 1;
+    return static_cast<int>(std::min<std::int64_t>(256, blocks_for(count, LOSS_AHEAD * LOSS_THREADS)));
+}
+
+int launch_mse_loss(const float* pred, const float* target, float* loss, std::int64_t count, double* partials,
+                    hipStream_t stream) {
+    const int groups = partials ? mse_loss_groups(count) : 1;
+    if (groups == 1) partials = nullptr;
+    launch(mse_loss_kernel, groups, LOSS_THREADS, 0, stream, pred, target, loss, partials, count);
+    MFH_TRY(MFH_CHECK_LAUNCH("mse_loss", stream));
+    if (groups == 1) return OK;
+    launch(mse_finish_kernel, 1, LOSS_THREADS, 0, stream, partials, groups, loss, count);
+    return MFH_CHECK_LAUNCH("mse_finish", stream);
 }
 
 int launch_mse_grad(const float* pred, const float* target, const float* seed, float* grad, std::int64_t count,
@@ -123,7 +216,7 @@ int launch_mse_grad(const float* pred, const float* target, const float* seed, f
 
 int launch_column_sums(const float* src, float* out, std::int64_t rows, std::int64_t cols, hipStream_t stream) {
     if (cols == 0) return OK;
-    launch(column_sums_kernel, blocks_for(cols, HEAD_THREADS), HEAD_THREADS, 0, stream, src, out, rows, cols);
+    launch(column_sums_kernel, blocks_for(cols, COLUMN_SPAN), COLUMN_SPAN * COLUMN_GROUPS, 0, stream, src, out, rows, cols);
     return MFH_CHECK_LAUNCH("column_sums", stream);
 }
 

@@ -318,7 +318,14 @@ def mse_loss_forward(pred, target):
     if pred.shape != target.shape:
         raise ValueError("pred and target must have the same shape")
     loss = torch.empty((), dtype=torch.float32, device=pred.device)
-    native._call("mfh_mse_loss", pred.data_ptr(), target.data_ptr(), loss.data_ptr(), pred.numel(), native._stream())
+    count = pred.numel()
+    partials = native._library().mfh_mse_loss_workspace(count)
+    if partials > 0:
+        workspace = torch.empty((partials,), dtype=torch.float64, device=pred.device)
+        native._call("mfh_mse_loss_split", pred.data_ptr(), target.data_ptr(), loss.data_ptr(), count,
+                     workspace.data_ptr(), partials, native._stream())
+    else:
+        native._call("mfh_mse_loss", pred.data_ptr(), target.data_ptr(), loss.data_ptr(), count, native._stream())
     return loss
 
 

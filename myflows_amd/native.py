@@ -130,6 +130,8 @@ _SIGNATURES = {
     "mfh_plane_mean": ("i", "ppqip"),
     "mfh_plane_mean_backward": ("i", "ppqiip"),
     "mfh_mse_loss": ("i", "pppqp"),
+    "mfh_mse_loss_workspace": ("q", "q"),
+    "mfh_mse_loss_split": ("i", "pppqpqp"),
     "mfh_mse_loss_backward": ("i", "ppppqip"),
     "mfh_column_sums": ("i", "ppqqp"),
 }

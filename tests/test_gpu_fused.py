@@ -202,6 +202,43 @@ def test_mse_loss_and_gradient_match_the_oracle(shape):
     np.testing.assert_array_equal(host(out), base + rp.mse_backward(pred, target))
 
 
+@pytest.mark.parametrize("hw", ((3, 5), (4, 4), (9, 13), (1, 127), (8, 16), (1, 255), (16, 16), (29, 39)))
+def test_plane_means_at_the_lane_counts_edges(hw):
+    """Every lane count per plane (1 below 16 elements, 16 below 128, 64) at its remainders. FP64 sums in
+    any order are within hw * 2^-53 of each other, so the rounded means differ by at most one ulp."""
+    print("plane means", hw, flush=True)
+    x = np.random.default_rng(41).normal(size=(3, 37, *hw)).astype(np.float32)
+    got, ref = host(fused.global_avg_pool_forward(gpu(x))), rp.gap_forward(x)
+    assert np.all(np.abs(got - ref) <= np.spacing(np.abs(ref)))
+    x[1, 2, 0, 1], x[2, 5, -1, -1] = np.inf, np.nan
+    got = host(fused.global_avg_pool_forward(gpu(x)))
+    assert got[1, 2] == np.inf and np.isnan(got[2, 5]) and np.isfinite(got).sum() == got.size - 2
+
+
+@pytest.mark.parametrize("count", (1, 1023, 8193, 32768, 32769, 256000, 2 ** 21 + 2 ** 13 + 5))
+def test_mse_loss_on_one_and_on_several_workgroups(count):
+    """Around the switch to several workgroups and past their largest number; a sum of positive FP64
+    terms in any order is within count * 2^-53 of the exact one: one float32 ulp after the rounding."""
+    print("mse workgroups", count, flush=True)
+    rng = np.random.default_rng(42)
+    pred, target = (rng.normal(size=(count,)).astype(np.float32) for _ in range(2))
+    loss, ref = host(fused.mse_loss_forward(gpu(pred), gpu(target))), rp.mse_forward(pred, target)
+    assert abs(float(loss) - float(ref)) <= np.spacing(np.float32(ref)), (loss, ref)
+    pred[-1] = np.nan
+    assert np.isnan(host(fused.mse_loss_forward(gpu(pred), gpu(target))))
+
+
+@pytest.mark.parametrize("rows,cols", ((0, 5), (1, 1), (15, 63), (16, 64), (17, 65), (128, 64), (129, 130), (1000, 10)))
+def test_column_sums_at_the_row_groups_edges(rows, cols):
+    """The 16 runs of rows, empty and ragged ones among them (cancelling sums: compared in absolute terms
+    with the FP64 sum's own error plus the final rounding)."""
+    print("column sums", rows, cols, flush=True)
+    g = np.random.default_rng(43).normal(size=(rows, cols)).astype(np.float32)
+    got, exact = host(fused.column_sums(gpu(g))), g.astype(np.float64).sum(axis=0)
+    bound = np.spacing(np.abs(exact).astype(np.float32)) + 2.0 ** -52 * rows * np.abs(g).sum(axis=0)
+    assert np.all(np.abs(got - exact) <= bound)
+
+
 def test_mse_of_no_elements_is_nan_like_the_oracle():
     empty = np.zeros((0, 2), dtype=np.float32)
     with np.errstate(invalid="ignore", divide="ignore"), pytest.warns(RuntimeWarning):
