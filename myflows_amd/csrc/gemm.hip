@@ -164,13 +164,37 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_grouped_
 // C = act((float)(((0.0 + p0) + p1) + ... + p[S-1]) [+ bias]) with the FP64 sum in slice order,
 // the bias (per column or per row) added in FP32 after the rounding, stored dense (row * ldc + col)
 // or segmented like the GEMM's own epilogue (C = C + that when p.accumulate).
-__device__ __forceinline__ void finish_output(const GemmParams& p, float* C, long long i, double s) {
-    const int row = static_cast<int>(i / p.N), col = static_cast<int>(i % p.N);
+__device__ __forceinline__ void finish_output(const GemmParams& p, float* C, int row, int col, double s) {
     float v = static_cast<float>(s);
     if (p.bias_mode == BIAS_COLUMN) v += p.bias[col];
     else if (p.bias_mode == BIAS_ROW) v += p.bias[row];
     if (p.residual) v = v + p.residual[output_offset(p, row, col)];
     write_output(p, C, row, col, activate(v, p.act, p.alpha));
+}
+
+// Row and column of output i by the multiply-and-shift division of columns = FastDiv(N) (a product
+// has at most INDEX_LIMIT outputs, so i fits an int). A 64-bit division and remainder per output
+// are some 200 vector instructions, which bounded the reductions.
+__device__ __forceinline__ void finish_output(const GemmParams& p, const FastDiv& columns, float* C, long long i,
+                                              double s) {
+    int col;
+    const int row = columns.divmod(static_cast<int>(i), col);
+    finish_output(p, C, row, col, s);
+}
+
+// Outputs i .. i + 3: one division, and the columns counted on from it.
+__device__ __forceinline__ void finish_quad(const GemmParams& p, const FastDiv& columns, float* C, long long i,
+                                            const double (&s)[4]) {
+    int col;
+    int row = columns.divmod(static_cast<int>(i), col);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        finish_output(p, C, row, col, s[r]);
+        if (++col == p.N) {
+            col = 0;
+            ++row;
+        }
+    }
 }
 
 constexpr int REDUCE_AHEAD = 8;  // slices loaded before they are added
@@ -192,7 +216,7 @@ __device__ __forceinline__ void finish_row(const GemmParams& p, long long t) {
 // One thread per output; the loads of REDUCE_AHEAD slices are issued before their additions, which
 // still run one at a time in slice order.
 __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ partial, float* __restrict__ C,
-                                                           GemmParams p, int slices) {
+                                                           GemmParams p, int slices, FastDiv columns) {
     raise_wave_priority();
     const long long i = blockIdx.x * 256LL + threadIdx.x, total = static_cast<long long>(p.M) * p.N;
     if (p.row_out) finish_row(p, i);
@@ -207,13 +231,14 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restri
         for (int u = 0; u < REDUCE_AHEAD; ++u) s += static_cast<double>(part[u]);
     }
     for (; z < slices; ++z) s += static_cast<double>(partial[z * total + i]);
-    finish_output(p, C, i, s);
+    finish_output(p, columns, C, i, s);
 }
 
 // Four adjacent outputs per thread with 16-byte loads (M * N % 4 == 0, aligned partials); the same
 // slice-order FP64 sums as split_reduce_kernel.
 __global__ __launch_bounds__(256) void split_reduce_vec4_kernel(const float* __restrict__ partial,
-                                                                float* __restrict__ C, GemmParams p, int slices) {
+                                                                float* __restrict__ C, GemmParams p, int slices,
+                                                                FastDiv columns) {
     raise_wave_priority();
     const long long q = blockIdx.x * 256LL + threadIdx.x, total = static_cast<long long>(p.M) * p.N;
     if (p.row_out) finish_row(p, q);
@@ -241,10 +266,8 @@ __global__ __launch_bounds__(256) void split_reduce_vec4_kernel(const float* __r
         s2 += static_cast<double>(part.z);
         s3 += static_cast<double>(part.w);
     }
-    finish_output(p, C, q * 4, s0);
-    finish_output(p, C, q * 4 + 1, s1);
-    finish_output(p, C, q * 4 + 2, s2);
-    finish_output(p, C, q * 4 + 3, s3);
+    const double sums[4] = {s0, s1, s2, s3};
+    finish_quad(p, columns, C, q * 4, sums);
 }
 
 // Many slices over few outputs (a dW product split over the pixels): thread (q, g) of a block of
@@ -253,7 +276,7 @@ __global__ __launch_bounds__(256) void split_reduce_vec4_kernel(const float* __r
 // result does not depend on timing (it is the slice-order sum regrouped, not its bits).
 constexpr int REDUCE_GROUPS = 8, GROUP_QUADS = 32;
 __global__ __launch_bounds__(REDUCE_GROUPS* GROUP_QUADS) void split_reduce_grouped_kernel(
-    const float* __restrict__ partial, float* __restrict__ C, GemmParams p, int slices) {
+    const float* __restrict__ partial, float* __restrict__ C, GemmParams p, int slices, FastDiv columns) {
     __shared__ double group_sum[REDUCE_GROUPS][GROUP_QUADS][4];
     const long long t = blockIdx.x * static_cast<long long>(REDUCE_GROUPS * GROUP_QUADS) + threadIdx.x;
     if (p.row_out) finish_row(p, t);
@@ -291,14 +314,15 @@ __global__ __launch_bounds__(REDUCE_GROUPS* GROUP_QUADS) void split_reduce_group
     group_sum[g][qi][2] = s2;
     group_sum[g][qi][3] = s3;
     __syncthreads();
-    if (g != 0 || q >= stride) return;
+    // Thread i < 4 * GROUP_QUADS finishes output i of the block (group 0's threads finishing four each
+    // in turn left the block's other waves idle).
+    const int output = threadIdx.x / 4, r = threadIdx.x % 4;
+    const long long first = static_cast<long long>(blockIdx.x) * GROUP_QUADS + output;
+    if (output >= GROUP_QUADS || first >= stride) return;
+    double sum = group_sum[0][output][r];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        double sum = group_sum[0][qi][r];
-#pragma unroll
-        for (int h = 1; h < REDUCE_GROUPS; ++h) sum += group_sum[h][qi][r];
-        finish_output(p, C, q * 4 + r, sum);
-    }
+    for (int h = 1; h < REDUCE_GROUPS; ++h) sum += group_sum[h][output][r];
+    finish_output(p, columns, C, first * 4 + r, sum);
 }
 
 using GemmFn = void (*)(GemmParams);
@@ -482,11 +506,13 @@ int launch_split_reduce(const float* partial, float* c, GemmParams p, int slices
     p.row_slices = slices;
     if (outputs % 4 == 0 && aligned16(partial)) {
         const std::int64_t threads = std::max<std::int64_t>(outputs / 4, 64LL * p.row_count);
-        launch(split_reduce_vec4_kernel, blocks_for(threads, 256), 256, 0, stream, partial, c, p, slices);
+        launch(split_reduce_vec4_kernel, blocks_for(threads, 256), 256, 0, stream, partial, c, p, slices,
+           FastDiv(std::max(1, p.N)));
         return MFH_CHECK_LAUNCH("split_reduce_vec4", stream);
     }
     const std::int64_t threads = std::max<std::int64_t>(outputs, 64LL * p.row_count);
-    launch(split_reduce_kernel, blocks_for(threads, 256), 256, 0, stream, partial, c, p, slices);
+    launch(split_reduce_kernel, blocks_for(threads, 256), 256, 0, stream, partial, c, p, slices,
+           FastDiv(std::max(1, p.N)));
     return MFH_CHECK_LAUNCH("split_reduce", stream);
 }
 
@@ -505,7 +531,8 @@ int split_reduce_grouped(const float* partial, float* c, const GemmEpilogue& e, 
     if (outputs % 4 != 0 || !aligned16(partial)) return launch_split_reduce(partial, c, p, slices, stream);
     const std::int64_t blocks = std::max<std::int64_t>(blocks_for(outputs / 4, GROUP_QUADS),
                                                        blocks_for(64LL * p.row_count, REDUCE_GROUPS * GROUP_QUADS));
-    launch(split_reduce_grouped_kernel, blocks, REDUCE_GROUPS * GROUP_QUADS, 0, stream, partial, c, p, slices);
+    launch(split_reduce_grouped_kernel, blocks, REDUCE_GROUPS * GROUP_QUADS, 0, stream, partial, c, p, slices,
+           FastDiv(std::max(1, p.N)));
     return MFH_CHECK_LAUNCH("split_reduce_grouped", stream);
 }
 
