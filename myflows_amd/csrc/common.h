@@ -431,15 +431,21 @@ struct AdamScalars {
 };
 int launch_adam(const AdamTensor* tensors, int count, const AdamScalars& s, hipStream_t stream);
 
+// ---- gemm_small.hip -------------------------------------------------------------------------
+// Whether the one-launch kernel for small products takes a product with a dense output, and its
+// launch (p: operands, sizes and epilogue).
+bool gemm_takes_small(int M, int N, int K);
+int launch_gemm_small(GemmParams p, bool trans_a, bool trans_b, hipStream_t stream);
+
 // ---- head.hip -------------------------------------------------------------------------------
 // y[p] = float(FP64 mean of x[p * hw .. p * hw + hw))
 int launch_plane_mean(const float* x, float* y, std::int64_t planes, int hw, hipStream_t stream);
 // dx[p * hw + i] (+)= dy[p] / float(hw)
 int launch_plane_mean_backward(const float* dy, float* dx, std::int64_t planes, int hw, bool add, hipStream_t stream);
-// loss[0] = float(FP64 sum of float32 (pred - target)^2 / count), NaN when count is 0
 // The workgroups that form the loss of count elements; from two on they need that many doubles of
 // partials (without them one workgroup does it).
 int mse_loss_groups(std::int64_t count);
+// loss[0] = float(FP64 sum of float32 (pred - target)^2 / count), NaN when count is 0
 int launch_mse_loss(const float* pred, const float* target, float* loss, std::int64_t count, double* partials,
                     hipStream_t stream);
 // grad (+)= seed[0] * ((2 * (pred - target)) / float(count)), float32 in that order

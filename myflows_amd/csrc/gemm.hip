@@ -577,10 +577,15 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(GemmParams p, int tran
     }
 }
 
+// Whether gemm_launch may run the problem on a kernel of its own beside the tiles: the automatic plan
+// of one product with a dense output.
+bool plain_auto(int engine, int batch, const GemmEpilogue& e) {
+    return engine == 1 && batch == 1 && e.segment == 0 && e.taps == 0 && e.lattice_w == 0 && !e.residual;
+}
+
 // Whether gemm_launch runs the problem on gemm_skinny_kernel.
 bool takes_skinny(int engine, int batch, int N, const GemmEpilogue& e) {
-    return engine == 1 && batch == 1 && N <= SKINNY_N && e.segment == 0 && e.taps == 0 && e.lattice_w == 0 &&
-           !e.residual;
+    return plain_auto(engine, batch, e) && N <= SKINNY_N;
 }
 
 }  // namespace
@@ -606,6 +611,16 @@ int gemm_launch(int engine, hipStream_t stream, const GemmOperands& o, const Gem
         p.k_chunk = K;
         launch(gemm_skinny_kernel, blocks_for(M, 4), 256, 0, stream, p, o.trans_a ? 1 : 0, o.trans_b ? 1 : 0);
         return MFH_CHECK_LAUNCH("gemm_skinny", stream);
+    }
+    if (plain_auto(engine, o.batch, e) && gemm_takes_small(M, N, K)) {
+        GemmParams p = epilogue_params(e, M, N, o.ldc);
+        p.A = o.a;
+        p.B = o.b;
+        p.C = o.c;
+        p.K = K;
+        p.lda = o.lda;
+        p.ldb = o.ldb;
+        return launch_gemm_small(p, o.trans_a, o.trans_b, stream);
     }
     GemmPlan plan;
     MFH_TRY(gemm_plan_from_engine(engine, M, N, K, &plan, o.batch));

@@ -289,3 +289,47 @@ def test_k_grouped_tile_is_the_group_order_sum_of_one_group_products(layout, m, 
     assert torch.equal(got, expected)
     got = native.gemm(a, b, bias, trans_a=trans_a, trans_b=trans_b, plan=("64x64k2", 1))
     assert torch.equal(got, expected + bias)
+
+
+@pytest.mark.parametrize("layout", ("NN", "NT", "TN"))
+@pytest.mark.parametrize("m,n,k", ((1, 9, 1), (32, 32, 16), (33, 31, 17), (31, 65, 127), (64, 96, 128), (100, 130, 257),
+                                   (256, 1000, 512), (512, 1024, 129), (45, 33, 2047), (17, 40, 2048)))
+def test_small_products_at_the_edges_of_their_tiles_and_runs(layout, m, n, k):
+    """gemm_small.hip: 32 x 32 tiles, eight runs of K in 16-deep steps, idle and ragged runs, both load
+    widths. Each output is k float32 multiply-adds in some order: |error| <= (k + 16) * 2^-24 * |A||B|."""
+    print("small", layout, m, n, k, flush=True)
+    rng = np.random.default_rng(k)
+    a, b = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(k, n)).astype(np.float32)
+    bias = rng.normal(size=(n,)).astype(np.float32)
+    ta, tb = layout[0] == "T", layout[1] == "T"
+    dev = [torch.as_tensor(np.ascontiguousarray(x), device="cuda") for x in (a.T if ta else a, b.T if tb else b, bias)]
+    got = native.gemm(dev[0], dev[1], dev[2], trans_a=ta, trans_b=tb).cpu().numpy()
+    exact = a.astype(np.float64) @ b.astype(np.float64) + bias
+    bound = (k + 16) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b) + np.abs(bias))
+    assert np.all(np.abs(got - exact) <= bound)
+
+
+def test_small_products_keep_infinities_to_their_own_rows_and_columns():
+    a, b = np.ones((40, 37), np.float32), np.ones((37, 50), np.float32)
+    a[39, 36], b[36, 49] = np.inf, 2.0
+    got = native.gemm(torch.as_tensor(a, device="cuda"), torch.as_tensor(b, device="cuda")).cpu().numpy()
+    assert np.all(np.isinf(got[39])) and np.isfinite(got[:39]).all() and np.all(got[:39, :49] == 37)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", ((131, 67, 61), (300, 261, 1030), (65, 129, 31)))
+def test_every_tile_reads_unaligned_rows(layout, m, n, k):
+    """Rows that start off 16-byte boundaries (odd sizes, and a base one float off), whole and ragged
+    stages, on every tile of the catalogue."""
+    trans_a, trans_b = LAYOUTS[layout]
+    a, b, exact, magnitude = operands(np.random.default_rng(5), m, n, k, trans_a, trans_b)
+
+    def shifted(x):
+        held = torch.empty(x.size + 1, dtype=torch.float32, device="cuda")
+        held[1:] = gpu(x).reshape(-1)
+        return held[1:].view(x.shape)
+
+    for tile in range(len(native.tile_catalog())):
+        print("unaligned", layout, (m, n, k), tile, flush=True)
+        got = host(native.gemm(shifted(a), shifted(b), trans_a=trans_a, trans_b=trans_b, plan=(tile, 1)))
+        assert np.all(np.abs(got - exact) <= gamma_k(k) * magnitude + EPS32 * np.abs(exact))
