@@ -5,8 +5,9 @@
 // 16-deep stages with a barrier each, and a 100 x 130 output over K = 257 is six 64 x 64 tiles of
 // nine stages, about 1 us a stage. Here a wave reads its operands straight into the MFMA's lanes
 // (no LDS, no barrier, two 16-deep steps in flight), K is shared by eight waves of the same
-// workgroup, and the eight partial tiles are added through LDS in wave order: one launch, no
-// workspace, each output summed in one fixed order.
+// workgroup, and the eight partial tiles are added through LDS in wave order in FP64 and rounded
+// once (the automatic plan split many of these products, and its slices are summed so): one launch,
+// no workspace, each output summed in one fixed order.
 #include <algorithm>
 
 #include "common.h"
@@ -98,9 +99,11 @@ __global__ __launch_bounds__(SMALL_THREADS) void gemm_small_kernel(GemmParams p)
     for (int i = threadIdx.x; i < SMALL_TILE * SMALL_TILE; i += SMALL_THREADS) {
         const int row = m0 + i / SMALL_TILE, col = n0 + i % SMALL_TILE;
         if (row >= p.M || col >= p.N) continue;
-        float v = partial[0][i];
+        // FP64, rounded once, as the reduction of a split plan adds its slices.
+        double sum = static_cast<double>(partial[0][i]);
 #pragma unroll
-        for (int w = 1; w < SMALL_WAVES; ++w) v += partial[w][i];
+        for (int w = 1; w < SMALL_WAVES; ++w) sum += static_cast<double>(partial[w][i]);
+        float v = static_cast<float>(sum);
         if (p.bias_mode == BIAS_COLUMN) v += p.bias[col];
         else if (p.bias_mode == BIAS_ROW) v += p.bias[row];
         write_output(p, p.C, row, col, activate(v, p.act, p.alpha));

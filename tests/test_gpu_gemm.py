@@ -309,6 +309,27 @@ def test_small_products_at_the_edges_of_their_tiles_and_runs(layout, m, n, k):
     assert np.all(np.abs(got - exact) <= bound)
 
 
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", ((100, 130, 257), (33, 65, 512), (256, 512, 1000), (128, 128, 1024), (500, 1000, 511)),
+                         ids=str)
+def test_small_products_add_their_runs_of_k_in_fp64(layout, m, n, k):
+    """The eight runs of K (whole 16-deep steps each) are the one-group tiles' products over those
+    ranges, added in run order in FP64 and rounded once, as a split plan's slices are; the bias is added
+    after the rounding. Bit for bit."""
+    print("small runs", layout, m, n, k, flush=True)
+    trans_a, trans_b = LAYOUTS[layout]
+    rng = np.random.default_rng(9)
+    a, b, _, _ = operands(rng, m, n, k, trans_a, trans_b)
+    a, b, bias = gpu(a), gpu(b), gpu(rng.standard_normal(n).astype(np.float32))
+    run = -(-(-(-k // 8)) // 16) * 16
+    cut = lambda x, lo, hi, k_first: (x[lo:hi] if k_first else x[:, lo:hi]).contiguous()
+    parts = [native.gemm(cut(a, lo, min(k, lo + run), trans_a), cut(b, lo, min(k, lo + run), not trans_b),
+                         trans_a=trans_a, trans_b=trans_b, plan=("64x64", 1)) for lo in range(0, k, run)]
+    expected = gpu(fp64_slice_sum(np.stack([host(part) for part in parts])))
+    assert torch.equal(native.gemm(a, b, trans_a=trans_a, trans_b=trans_b), expected)
+    assert torch.equal(native.gemm(a, b, bias, trans_a=trans_a, trans_b=trans_b), expected + bias)
+
+
 def test_small_products_keep_infinities_to_their_own_rows_and_columns():
     a, b = np.ones((40, 37), np.float32), np.ones((37, 50), np.float32)
     a[39, 36], b[36, 49] = np.inf, 2.0
