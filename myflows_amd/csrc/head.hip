@@ -13,6 +13,7 @@
 #include <cstdint>
 
 #include "common.h"
+#include "plane_walk.h"
 
 namespace mfh {
 namespace {
@@ -32,15 +33,16 @@ __global__ __launch_bounds__(HEAD_THREADS) void plane_mean_kernel(const float* _
     const int lane = threadIdx.x % LANES;
     const float* __restrict__ src = x + p * hw;
     double s = 0.0;
-    int i = lane;
-    for (; i + 3 * LANES < hw; i += 4 * LANES) {
-        float v[4];
+    walk_plane<LANES, 4>(
+        lane, hw,
+        [&](unsigned i) {
+            float v[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = src[i + u * LANES];
+            for (int u = 0; u < 4; ++u) v[u] = src[i + u * LANES];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) s += static_cast<double>(v[u]);
-    }
-    for (; i < hw; i += LANES) s += static_cast<double>(src[i]);
+            for (int u = 0; u < 4; ++u) s += static_cast<double>(v[u]);
+        },
+        [&](unsigned i) { s += static_cast<double>(src[i]); });
 #pragma unroll
     for (int offset = LANES / 2; offset > 0; offset >>= 1) s += __shfl_xor(s, offset, LANES);
     if (lane == 0) y[p] = static_cast<float>(s / static_cast<double>(hw));

@@ -56,6 +56,32 @@ def test_adam_table_layout_matches_the_header(tmp_path):
     assert c_layout == [ctypes.sizeof(t), t.size.offset, t.lr.offset, t.bias_correction2.offset]
 
 
+@pytest.mark.parametrize("lanes", (1, 16, 64))
+def test_plane_mean_lanes_visit_each_element_once_up_to_the_largest_plane(tmp_path, lanes):
+    """The walk of a lane over its plane (csrc/plane_walk.h, compiled for the host): every index it reads
+    lies in the plane and follows the last by `lanes`, and it stops at the plane's end, planes of up to
+    2^31 - 1 elements (the largest the entry point takes) included."""
+    counts = [1, 15, 16, 127, 128, 255, 1131] + ([2 ** 31 - 1 - e for e in (0, 1, 63, 192, 256)] if lanes == 64 else [])
+    probe = tmp_path / "probe.cpp"
+    probe.write_text(
+        '#include <cstdlib>\n#include <initializer_list>\n#define __host__\n#define __device__\n#include "plane_walk.h"\n'
+        f"constexpr unsigned LANES = {lanes};\n"
+        "int main(int, char** argv) {\n"
+        "  const unsigned count = std::strtoul(argv[1], nullptr, 10);\n"
+        "  for (unsigned lane : {0u, LANES / 2, LANES - 1}) {\n"
+        "    long long next = lane; bool ok = true;\n"
+        "    auto one = [&](long long i) { ok = ok && i == next && i < count; next += LANES; };\n"
+        "    mfh::walk_plane<LANES, 4>(lane, count, [&](unsigned i) {\n"
+        "      for (int u = 0; u < 4 && ok; ++u) one(static_cast<long long>(i) + u * LANES);\n"
+        "      if (!ok) std::exit(1); }, [&](unsigned i) { one(i); if (!ok) std::exit(1); });\n"
+        "    if (next < count) return 2;\n"
+        "  }\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-I", str(HEADER.parents[1] / "myflows_amd" / "csrc"), str(probe), "-o",
+                    str(tmp_path / "probe")], check=True)
+    for count in counts:
+        assert subprocess.run([str(tmp_path / "probe"), str(count)], timeout=60).returncode == 0, count
+
+
 def test_tile_catalogue_and_plan_codes():
     catalogue = native.tile_catalog()
     assert catalogue["128x128"][0] == 0
