@@ -317,14 +317,18 @@ def mse_loss_forward(pred, target):
     pred, target = _f32(pred, "pred"), _f32(target, "target")
     if pred.shape != target.shape:
         raise ValueError("pred and target must have the same shape")
-    loss = torch.empty((), dtype=torch.float32, device=pred.device)
     count = pred.numel()
     partials = native._library().mfh_mse_loss_workspace(count)
     if partials > 0:
-        workspace = torch.empty((partials,), dtype=torch.float64, device=pred.device)
-        native._call("mfh_mse_loss_split", pred.data_ptr(), target.data_ptr(), loss.data_ptr(), count,
-                     workspace.data_ptr(), partials, native._stream())
+        # The workgroups' doubles lie behind the loss in its own storage: they live as long as the caller
+        # keeps the loss. A block of their own, freed on return, could be handed out on the current stream
+        # while the launches still run on the stream of a launch_stream block.
+        held = torch.empty((2 + 2 * partials,), dtype=torch.float32, device=pred.device)
+        loss = held[0]
+        native._call("mfh_mse_loss_split", pred.data_ptr(), target.data_ptr(), held.data_ptr(), count,
+                     held.data_ptr() + 8, partials, native._stream())
     else:
+        loss = torch.empty((), dtype=torch.float32, device=pred.device)
         native._call("mfh_mse_loss", pred.data_ptr(), target.data_ptr(), loss.data_ptr(), count, native._stream())
     return loss
 

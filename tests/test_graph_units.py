@@ -6,7 +6,7 @@ statistics that a second BN shares, leave the chain unfused. Graph building only
 import torch
 
 import myflows_amd as mf
-from myflows_amd import device
+from myflows_amd import device, fused, native
 from myflows_amd.resnet import BatchNorm2d
 
 
@@ -39,3 +39,27 @@ def test_materialize_intermediates_drops_the_fused_units_from_the_plan():
         assert graph._plan().groups
     finally:
         device.set_device(previous)
+
+
+def test_the_split_loss_keeps_its_scratch_as_long_as_the_loss(monkeypatch):
+    """The sums of the loss's workgroups must not go back to the allocator while a launch on another
+    stream (native.launch_stream) still uses them: they are part of the returned tensor's storage."""
+    calls = []
+    library = type("Library", (), {"mfh_mse_loss_workspace": staticmethod(lambda count: 32 if count > 32768 else 0)})
+    monkeypatch.setattr(fused, "_f32", lambda tensor, name: tensor)
+    monkeypatch.setattr(native, "_library", lambda: library)
+    monkeypatch.setattr(native, "_stream", lambda: 0)
+    monkeypatch.setattr(native, "_call", lambda *args: calls.append(args))
+    for count in (32768, 256000):
+        pred = torch.zeros(count)
+        loss = fused.mse_loss_forward(pred, pred)
+        assert loss.shape == () and loss.dtype == torch.float32 and loss.is_contiguous()
+        symbol, *args = calls[-1]
+        assert args[2] == loss.data_ptr() and args[3] == count
+        if count == 32768:
+            assert symbol == "mfh_mse_loss"
+            continue
+        scratch, doubles = args[4], args[5]
+        storage = loss.untyped_storage()
+        assert symbol == "mfh_mse_loss_split" and doubles == 32 and scratch % 8 == 0
+        assert loss.data_ptr() + 4 <= scratch and scratch + 8 * doubles <= storage.data_ptr() + storage.nbytes()
