@@ -7,8 +7,8 @@
 //   * loss = float(FP64 sum of float32 (d * d) / count), d = pred - target (float32 difference and
 //     square, as the operator's diff * diff)
 //   * its gradient g[i] (+)= seed * ((2 * d) / float(count))             (float32, in that order)
-//   * column sums out[j] = float(FP64 sum over rows of src[r, j]), 16 runs of rows, each in order, then in
-//     run order.
+//   * column sums out[j] = float(FP64 sum over rows of src[r, j]): in 1, 4 or 16 runs of rows, each in
+//     order, then in run order.
 #include <algorithm>
 #include <cstdint>
 
@@ -133,18 +133,16 @@ __global__ __launch_bounds__(HEAD_THREADS) void mse_grad_kernel(const float* __r
     grad[i] = add ? grad[i] + v : v;
 }
 
-// A workgroup of COLUMN_SPAN columns by COLUMN_GROUPS row groups: group g adds its run of rows in
-// order in FP64, eight loads in flight; the groups' sums are then added in group order through LDS.
-// Latency bounds it: one thread per column walked 256 rows of 1000 columns in 12.6 us.
-constexpr int COLUMN_SPAN = 64, COLUMN_GROUPS = 16;
-
-__global__ __launch_bounds__(COLUMN_SPAN* COLUMN_GROUPS) void column_sums_kernel(const float* __restrict__ src,
-                                                                                 float* __restrict__ out,
-                                                                                 long long rows, long long cols) {
-    __shared__ double group_sum[COLUMN_GROUPS][COLUMN_SPAN];
-    const int c = threadIdx.x % COLUMN_SPAN, g = threadIdx.x / COLUMN_SPAN;
-    const long long j = static_cast<long long>(blockIdx.x) * COLUMN_SPAN + c;
-    const long long per = (rows + COLUMN_GROUPS - 1) / COLUMN_GROUPS;
+// A workgroup of SPAN columns by GROUPS row groups: group g adds its run of rows in order in FP64, eight
+// loads in flight; the groups' sums are then added in group order through LDS.
+template <int GROUPS, int SPAN>
+__global__ __launch_bounds__(SPAN* GROUPS) void column_sums_kernel(const float* __restrict__ src,
+                                                                   float* __restrict__ out, long long rows,
+                                                                   long long cols) {
+    __shared__ double group_sum[GROUPS][SPAN];
+    const int c = threadIdx.x % SPAN, g = threadIdx.x / SPAN;
+    const long long j = static_cast<long long>(blockIdx.x) * SPAN + c;
+    const long long per = (rows + GROUPS - 1) / GROUPS;
     const long long last = min(rows, (g + 1) * per);
     double s = 0.0;
     if (j < cols) {
@@ -158,12 +156,14 @@ __global__ __launch_bounds__(COLUMN_SPAN* COLUMN_GROUPS) void column_sums_kernel
         }
         for (; r < last; ++r) s += static_cast<double>(src[r * cols + j]);
     }
-    group_sum[g][c] = s;
-    __syncthreads();
-    if (g != 0 || j >= cols) return;
+    if constexpr (GROUPS > 1) {
+        group_sum[g][c] = s;
+        __syncthreads();
+        if (g != 0) return;
 #pragma unroll
-    for (int h = 1; h < COLUMN_GROUPS; ++h) s += group_sum[h][c];
-    out[j] = static_cast<float>(s);
+        for (int h = 1; h < GROUPS; ++h) s += group_sum[h][c];
+    }
+    if (j < cols) out[j] = static_cast<float>(s);
 }
 
 }  // namespace
@@ -218,7 +218,18 @@ int launch_mse_grad(const float* pred, const float* target, const float* seed, f
 
 int launch_column_sums(const float* src, float* out, std::int64_t rows, std::int64_t cols, hipStream_t stream) {
     if (cols == 0) return OK;
-    launch(column_sums_kernel, blocks_for(cols, COLUMN_SPAN), COLUMN_SPAN * COLUMN_GROUPS, 0, stream, src, out, rows, cols);
+    // Few rows: one thread a column, whose loads are in flight in a few rounds (groups would leave most of
+    // their block idle: 8 x 1000000 4.0 us, by 4 groups 9.6, by 16 26). More rows: a column's chain of loads
+    // bounds it, and groups share it, 16 of them while the columns alone do not fill the GPU (256 x 1000
+    // 6.4 us by one thread, 2.9 by 4 groups, 2.5 by 16; 2048 x 4096 44 / 12.5 / 7.1), 4 from 32769 columns
+    // on (64 x 100000 4.5 / 3.2 / 7.1, 256 x 65536 14.1 / 11.0 / 10.8).
+    const auto run = [&](auto kernel, int groups, int span) {
+        launch(kernel, blocks_for(cols, span), groups * span, 0, stream, src, out, rows, cols);
+    };
+    const bool wide = cols > 32768;
+    if (rows < (wide ? 64 : 48)) run(column_sums_kernel<1, 256>, 1, 256);
+    else if (wide) run(column_sums_kernel<4, 64>, 4, 64);
+    else run(column_sums_kernel<16, 64>, 16, 64);
     return MFH_CHECK_LAUNCH("column_sums", stream);
 }
 

@@ -228,10 +228,12 @@ def test_mse_loss_on_one_and_on_several_workgroups(count):
     assert np.isnan(host(fused.mse_loss_forward(gpu(pred), gpu(target))))
 
 
-@pytest.mark.parametrize("rows,cols", ((0, 5), (1, 1), (15, 63), (16, 64), (17, 65), (128, 64), (129, 130), (1000, 10)))
+@pytest.mark.parametrize("rows,cols", ((0, 5), (1, 1), (15, 63), (16, 64), (17, 65), (128, 64), (129, 130),
+                                       (1000, 10), (17, 257), (47, 65), (48, 64), (49, 130), (47, 32768),
+                                       (48, 32768), (48, 32769), (63, 32769), (64, 32769), (131, 32771)))
 def test_column_sums_at_the_row_groups_edges(rows, cols):
-    """The 16 runs of rows, empty and ragged ones among them (cancelling sums: compared in absolute terms
-    with the FP64 sum's own error plus the final rounding)."""
+    """The 1, 4 and 16 runs of rows at the limits between them, empty and ragged ones among them
+    (cancelling sums: compared in absolute terms with the FP64 sum's own error plus the final rounding)."""
     print("column sums", rows, cols, flush=True)
     g = np.random.default_rng(43).normal(size=(rows, cols)).astype(np.float32)
     got, exact = host(fused.column_sums(gpu(g))), g.astype(np.float64).sum(axis=0)
