@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "tile_loader.h"
 
 namespace mfh {
 
@@ -59,68 +60,6 @@ struct MfmaShape {
     static constexpr int B_SIZE = TB ? BN * LDB_S : BK * LDB_S;
     static constexpr int STAGE = A_SIZE + B_SIZE;
     static_assert(BK % 8 == 0, "each lane half consumes groups of four k");
-};
-
-// Four floats at any float's address (the hardware's 16-byte loads need 4-byte alignment only).
-typedef float UnalignedQuad __attribute__((ext_vector_type(4), aligned(4)));
-
-// A ROWS x COLS tile whose COLS dimension is contiguous in global memory (row stride ld), staged
-// through registers in quads: load() issues the global reads, store() writes them to LDS. VEC: every
-// row's start is 16-byte aligned and col_limit a multiple of 4. Otherwise (odd sizes) a tile that
-// lies inside the columns still takes 16-byte loads, from wherever its rows start; only a tile across
-// col_limit, the same for the whole workgroup, reads single floats. (Single floats everywhere made four
-// times the load instructions: 1531 x 1000 over K = 777, transposed B, 41.3 -> 37.9 us, the same bits.)
-template <int ROWS, int COLS, int THREADS, bool VEC>
-struct TileLoader {
-    static_assert(COLS % 4 == 0, "whole quads per row");
-    static constexpr int ELEMS = ROWS * COLS / 4;
-    static constexpr int PER_THREAD = (ELEMS + THREADS - 1) / THREADS;
-    static constexpr int VCOLS = COLS / 4;
-    float4 v[PER_THREAD];
-
-    __device__ __forceinline__ void load(const float* __restrict__ base, int ld, int row0, int row_limit, int col0,
-                                         int col_limit, int tid) {
-        const bool inside = col0 + COLS <= col_limit;
-        if (VEC || inside) {
-#pragma unroll
-            for (int i = 0; i < PER_THREAD; ++i) {
-                const int f = tid + i * THREADS;
-                const int row = row0 + f / VCOLS, col = col0 + (f % VCOLS) * 4;
-                float4 value = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (f < ELEMS && row < row_limit && (VEC ? col < col_limit : true)) {
-                    const float* at = base + static_cast<long long>(row) * ld + col;
-                    if constexpr (VEC) {
-                        value = *reinterpret_cast<const float4*>(at);
-                    } else {
-                        const UnalignedQuad q = *reinterpret_cast<const UnalignedQuad*>(at);
-                        value = make_float4(q.x, q.y, q.z, q.w);
-                    }
-                }
-                v[i] = value;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < PER_THREAD; ++i) {
-                const int f = tid + i * THREADS;
-                const int row = row0 + f / VCOLS, col = col0 + (f % VCOLS) * 4;
-                const float* at = base + static_cast<long long>(row) * ld + col;
-                float e[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (f < ELEMS && row < row_limit && col + u < col_limit) e[u] = at[u];
-                v[i] = make_float4(e[0], e[1], e[2], e[3]);
-            }
-        }
-    }
-
-    template <int LD>
-    __device__ __forceinline__ void store(float* lds, int tid) const {
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-            const int f = tid + i * THREADS;
-            if (f < ELEMS) *reinterpret_cast<float4*>(lds + f / VCOLS * LD + f % VCOLS * 4) = v[i];
-        }
-    }
 };
 
 // Buffer loads (the raw buffer instructions of CDNA): a 128-bit resource in SGPRs holds the base

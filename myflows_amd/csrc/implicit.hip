@@ -354,7 +354,7 @@ __device__ __forceinline__ void implicit_forward_tile(const GemmParams& p, const
     // Chunked products (K a multiple of BK) read the kernel order with buffer loads too, two stages
     // ahead (two register slots of loaders); so do padded natural-order products, whose kernel is
     // a copy with its rows padded to whole stages (lda a multiple of BK, zeros past K).
-    using LoadA = std::conditional_t<AHEAD, BufferRowTile<BM, BK, S::THREADS>, TileLoader<BM, BK, S::THREADS, VA>>;
+    using LoadA = std::conditional_t<AHEAD, BufferRowTile<BM, BK, S::THREADS>, TileLoader<BM, BK, S::THREADS, VA, false>>;
     using LoadB = std::conditional_t<CHUNKED, GatherChunkRows<BN, S::THREADS>,
                                      std::conditional_t<PADDED, GatherPaddedRows<BN, S::THREADS>,
                                                         GatherFeatureRows<BN, S::THREADS>>>;

@@ -64,7 +64,8 @@ def test_plane_mean_lanes_visit_each_element_once_up_to_the_largest_plane(tmp_pa
     counts = [1, 15, 16, 127, 128, 255, 1131] + ([2 ** 31 - 1 - e for e in (0, 1, 63, 192, 256)] if lanes == 64 else [])
     probe = tmp_path / "probe.cpp"
     probe.write_text(
-        '#include <cstdlib>\n#include <initializer_list>\n#define __host__\n#define __device__\n#include "plane_walk.h"\n'
+        '#include <cstdlib>\n#include <initializer_list>\n#define __host__\n#define __device__\n'
+        '#include "plane_walk.h"\n'
         f"constexpr unsigned LANES = {lanes};\n"
         "int main(int, char** argv) {\n"
         "  const unsigned count = std::strtoul(argv[1], nullptr, 10);\n"
@@ -80,6 +81,103 @@ def test_plane_mean_lanes_visit_each_element_once_up_to_the_largest_plane(tmp_pa
                     str(tmp_path / "probe")], check=True)
     for count in counts:
         assert subprocess.run([str(tmp_path / "probe"), str(count)], timeout=60).returncode == 0, count
+
+
+TILE_LOADER_PROBE = r"""
+#include <sys/mman.h>
+#include <unistd.h>
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <initializer_list>
+#define __device__
+#define __forceinline__ inline
+struct alignas(4) float4 { float x, y, z, w; };
+inline float4 make_float4(float x, float y, float z, float w) { return {x, y, z, w}; }
+#include "tile_loader.h"
+
+// `count` floats that end (or start) at a page no access survives.
+struct Guarded {
+    char* map;
+    long long bytes, page;
+    float* data;
+    Guarded(long long count, bool at_end) : page(sysconf(_SC_PAGESIZE)) {
+        bytes = (count * 4 + page - 1) / page * page;
+        map = static_cast<char*>(mmap(nullptr, bytes + 2 * page, PROT_NONE,
+                                      MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0));
+        mprotect(map + page, bytes, PROT_READ | PROT_WRITE);
+        data = reinterpret_cast<float*>(map + page + (at_end ? bytes - count * 4 : 0));
+    }
+    ~Guarded() { munmap(map, bytes + 2 * page); }
+};
+
+template <int ROWS, int COLS, int THREADS, bool ROWS_K>
+void tile(const float* base, int ld, int row0, int rows, int col0, int cols, float* lds) {
+    for (int i = 0; i < ROWS * (COLS + 4); ++i) lds[i] = NAN;
+    for (int tid = 0; tid < THREADS; ++tid) {
+        mfh::TileLoader<ROWS, COLS, THREADS, false, ROWS_K> loader;
+        loader.load(base, ld, row0, rows, col0, cols, tid);
+        loader.template store<COLS + 4>(lds, tid);
+    }
+}
+
+template <int ROWS, int COLS, int THREADS, bool ROWS_K>
+int check() {
+    static float lds[ROWS * (COLS + 4)];
+    for (int rows : {1, 2, 3, 5, 16, 19, 20, 21, 33, 70})
+        for (int cols : {1, 2, 3, 4, 5, 15, 16, 17, 62, 63, 64, 65, 67, 130})
+            for (int pad : {0, 1, 3})
+                for (bool at_end : {false, true}) {
+                    const int ld = cols + pad;
+                    const long long count = static_cast<long long>(rows - 1) * ld + cols;
+                    Guarded held(count, at_end);
+                    for (long long i = 0; i < count; ++i) held.data[i] = static_cast<float>(1 + i);
+                    for (int row0 = 0; row0 < rows + 2 * ROWS; row0 += ROWS)  // the loads ahead pass the end
+                        for (int col0 = 0; col0 < cols + 2 * COLS; col0 += COLS) {
+                            if (ROWS_K ? col0 >= cols : row0 >= rows) continue;  // no workgroup there
+                            tile<ROWS, COLS, THREADS, ROWS_K>(held.data, ld, row0, rows, col0, cols, lds);
+                            for (int r = 0; r < ROWS; ++r)
+                                for (int c = 0; c < COLS; ++c) {
+                                    const int row = row0 + r, col = col0 + c;
+                                    const float got = lds[r * (COLS + 4) + c];
+                                    const bool in = row < rows && col < cols;
+                                    // Past the rows or columns that are not along k: reaches no output.
+                                    if (!in && (ROWS_K ? row < rows : row >= rows)) continue;
+                                    const float want = in ? held.data[static_cast<long long>(row) * ld + col] : 0.f;
+                                    if (got == want) continue;
+                                    printf("%d x %d ld %d at %d %d: %g not %g\n", rows, cols, ld, row, col, got, want);
+                                    return 1;
+                                }
+                        }
+                }
+    // Limits up to 2^31 - 1, the last tile (pages of zeros, mapped as they are touched).
+    for (int over : {0, 1, 2, 61}) {
+        const int limit = 2147483647 - over;
+        Guarded held(limit, true);
+        const int last = (limit - 1) / COLS * COLS;
+        tile<ROWS, COLS, THREADS, ROWS_K>(held.data, limit, 0, 1, last, limit, lds);
+        if (lds[0] != 0.f) return 1;
+    }
+    return 0;
+}
+
+int main() {
+    return check<16, 64, 256, true>() || check<64, 16, 256, false>() || check<16, 256, 512, true>() ||
+           check<32, 256, 1024, true>();
+}
+"""
+
+
+def test_tile_loads_read_no_byte_outside_the_operand(tmp_path):
+    """The tile loads of the GEMM (csrc/tile_loader.h, compiled for the host) at every kind of edge, on
+    operands that end or start at an inaccessible page: all terms in place, zeros where k ends, and no
+    access outside, for sizes up to 2^31 - 1."""
+    (tmp_path / "probe.cpp").write_text(TILE_LOADER_PROBE)
+    compiler = "/opt/rocm/llvm/bin/clang++" if Path("/opt/rocm/llvm/bin/clang++").exists() else "clang++"
+    subprocess.run([compiler, "-std=c++17", "-O1", "-fwrapv", "-I", str(HEADER.parents[1] / "myflows_amd" / "csrc"),
+                    str(tmp_path / "probe.cpp"), "-o", str(tmp_path / "probe")], check=True)
+    run = subprocess.run([str(tmp_path / "probe")], capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0, (run.returncode, run.stdout)
 
 
 def test_tile_catalogue_and_plan_codes():

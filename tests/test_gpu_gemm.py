@@ -354,3 +354,25 @@ def test_every_tile_reads_unaligned_rows(layout, m, n, k):
         print("unaligned", layout, (m, n, k), tile, flush=True)
         got = host(native.gemm(shifted(a), shifted(b), trans_a=trans_a, trans_b=trans_b, plan=(tile, 1)))
         assert np.all(np.abs(got - exact) <= gamma_k(k) * magnitude + EPS32 * np.abs(exact))
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", ((1, 1, 1), (2, 3, 2), (3, 70, 3), (70, 2, 3), (5, 6, 7), (66, 1, 130), (1, 67, 34),
+                                   (130, 131, 133), (257, 258, 67), (259, 33, 35)))
+def test_every_tile_reads_ragged_edges_exactly(layout, m, n, k):
+    """The last quad of a row (1, 2 or 3 floats over, and rows of fewer than four floats) on every tile:
+    small whole numbers, whose products are exact in float32, between NaNs that no output may see."""
+    trans_a, trans_b = LAYOUTS[layout]
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.integers(-8, 9, size=(m, k)), rng.integers(-8, 9, size=(k, n))
+
+    def guarded(x):
+        held = torch.full((x.size + 8,), float("nan"), dtype=torch.float32, device="cuda")
+        held[1:1 + x.size] = gpu(x.astype(np.float32)).reshape(-1)
+        return held[1:1 + x.size].view(x.shape)
+
+    da, db = guarded(a.T if trans_a else a), guarded(b.T if trans_b else b)
+    for tile in sorted(native.tile_catalog()):
+        print("ragged", layout, (m, n, k), tile, flush=True)
+        got = host(native.gemm(da, db, trans_a=trans_a, trans_b=trans_b, plan=(tile, 1)))
+        np.testing.assert_array_equal(got, (a @ b).astype(np.float32))
