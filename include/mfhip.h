@@ -319,11 +319,21 @@ MFH_API int mfh_gemm_tile_groups(int index);
  * 0 meant register double buffering and 2-4 a cp.async pipeline). */
 MFH_API int mfh_gemm_tile_stages(int index);
 
-/* Automatic tile and split-K slice count for C(M,N) over K.
+/* Automatic tile and split-K slice count for C(M,N) over K, where the MFMA tiles run it
+ * (mfh_gemm_kernel 0, and every product with a segmented output, as mfh_conv_forward's).
  * Replaces mf_gemm_plan, native_cublas.cpp:1635-1643. */
 MFH_API int mfh_gemm_plan(int M, int N, int K, int* tile, int* slices);
 
-/* Workspace floats the automatic plan uses (0 when it does not split), -1 on error.
+/* Which kernel engine 1 runs for C(M,N) over K with a dense output (mfh_gemm and mfh_gemm_noalloc,
+ * mfh_matmul's variant 4, the im2col path's products but the segmented forward): 0 the MFMA tiles by
+ * mfh_gemm_plan, 1 one wave per output row (N <= 8: lanes split K, a fixed butterfly adds them), 2 one
+ * launch of 32 x 32 tiles whose K eight waves share, their partial tiles added in FP64 in run order and
+ * rounded once (up to 512 such tiles, K up to 1024 below 257 of them and 512 above). 1 and 2 use no
+ * workspace. -1 on error. No counterpart in the reference. */
+MFH_API int mfh_gemm_kernel(int M, int N, int K);
+
+/* Workspace floats the automatic tile plan uses (0 when it does not split), -1 on error. A product that
+ * mfh_gemm_kernel takes off the tiles uses none of it.
  * Replaces mf_gemm_workspace, native_cublas.cpp:1659-1666. */
 MFH_API int64_t mfh_gemm_workspace(int M, int N, int K);
 
@@ -335,9 +345,8 @@ MFH_API int mfh_split_reduce(uint64_t partial, uint64_t c, int slices, int M, in
 
 /* C(M,N) = op(A) op(B) [+ bias(N)], row-major with leading dimensions lda/ldb/ldc. op(A) = A^T when
  * trans_a (A stored K x M), op(B) = B^T when trans_b (B stored N x K); not both. workspace may be
- * 0; with the plan's slices * M * N floats the engine splits K. bias needs ldc == N. Engine 1 with
- * N <= 8 runs one wave per output row (lanes split K, a fixed butterfly adds them); an explicit
- * plan code always runs the MFMA tiles.
+ * 0; with the plan's slices * M * N floats the engine splits K. bias needs ldc == N. Engine 1 runs the
+ * kernel that mfh_gemm_kernel names; an explicit plan code always runs the MFMA tiles.
  * Replaces mf_gemm, native_cublas.cpp:1672-1692. */
 MFH_API int mfh_gemm(int engine, int trans_a, int trans_b, uint64_t a, uint64_t b, uint64_t bias, uint64_t c, int M,
                      int N, int K, int lda, int ldb, int ldc, uint64_t workspace, int64_t workspace_floats,
@@ -351,7 +360,8 @@ MFH_API int mfh_gemm(int engine, int trans_a, int trans_b, uint64_t a, uint64_t 
  * to a fixed device array inside the library (MFH_GEMM_NOALLOC_SCRATCH_FLOATS floats per GPU, held
  * until the process ends). The call allocates nothing. A plan whose slices * M * N exceeds the
  * scratch is rejected with status 2 (the plan is the one mfh_gemm would run given a large enough
- * workspace: engine 1's automatic plan, or an explicit code). Every call on a GPU shares that GPU's
+ * workspace: engine 1's automatic plan, or an explicit code; what mfh_gemm_kernel takes off the tiles
+ * uses no scratch). Every call on a GPU shares that GPU's
  * scratch: calls that overlap in time on one GPU (on other streams or threads) race. Results are
  * bitwise those of mfh_gemm with the same engine and a workspace of the plan's size.
  * No counterpart in the reference (its mf_gemm always takes the caller's workspace). */

@@ -684,7 +684,8 @@ MFH_API int mfh_matmul(int variant, int tile, int accumulate, std::uint64_t a, s
     MFH_REQUIRE(!(variant == 1 || variant == 2) || tile == 16 || tile == 32, "tile must be 16 or 32");
     const hipStream_t s = as_stream(stream);
     if (variant == 4 && accumulate == 0) {
-        // The fp32 register variant is the MFMA engine in one pass over K, bias fused.
+        // The fp32 register variant is the MFMA engine without a workspace, bias fused: the tiles in one
+        // pass over K, or the kernel for small or narrow products.
         GemmOperands o{};
         o.M = M;
         o.N = N;
@@ -743,6 +744,14 @@ MFH_API int mfh_gemm_plan(int M, int N, int K, int* tile, int* slices) {
     *tile = plan.tile;
     *slices = plan.slices;
     return OK;
+}
+
+MFH_API int mfh_gemm_kernel(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0) {
+        MFH_FAIL(ERR_ARG, "GEMM dimensions must be positive");
+        return -1;
+    }
+    return gemm_auto_kernel(M, N, K);
 }
 
 MFH_API std::int64_t mfh_gemm_workspace(int M, int N, int K) {

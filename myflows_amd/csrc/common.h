@@ -218,9 +218,14 @@ struct GemmEpilogue {
 // plan's slices * M * N floats.
 int gemm_launch(int engine, hipStream_t stream, const GemmOperands& operands, const GemmEpilogue& epilogue,
                 float* workspace, std::int64_t workspace_floats);
+// The kernel gemm_launch runs for one problem with a dense output under engine 1: the tiles by the
+// automatic plan, one wave per output row (at most 8 columns), or the one-launch small tiles. The
+// last two take no workspace.
+constexpr int GEMM_KERNEL_TILES = 0, GEMM_KERNEL_SKINNY = 1, GEMM_KERNEL_SMALL = 2;
+int gemm_auto_kernel(int M, int N, int K);
 // Workspace floats gemm_launch uses for one problem with a plain epilogue (bias per column at
-// most) when it is given all it asks for: the plan's slices * M * N, or 0 (no split, or an output
-// of at most 8 columns under the automatic plan, which takes the one-wave-per-row kernel).
+// most) when it is given all it asks for: the plan's slices * M * N, or 0 (no split, or a product
+// that gemm_auto_kernel takes off the tiles).
 std::int64_t gemm_launch_workspace(int engine, int M, int N, int K);
 int split_reduce(const float* partial, float* c, int slices, int M, int N, int ldc, bool reference,
                  hipStream_t stream);

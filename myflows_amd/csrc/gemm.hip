@@ -588,15 +588,15 @@ bool plain_auto(int engine, int batch, const GemmEpilogue& e) {
     return engine == 1 && batch == 1 && e.segment == 0 && e.taps == 0 && e.lattice_w == 0 && !e.residual;
 }
 
-// Whether gemm_launch runs the problem on gemm_skinny_kernel.
-bool takes_skinny(int engine, int batch, int N, const GemmEpilogue& e) {
-    return plain_auto(engine, batch, e) && N <= SKINNY_N;
-}
-
 }  // namespace
 
+int gemm_auto_kernel(int M, int N, int K) {
+    if (N <= SKINNY_N) return GEMM_KERNEL_SKINNY;
+    return gemm_takes_small(M, N, K) ? GEMM_KERNEL_SMALL : GEMM_KERNEL_TILES;
+}
+
 std::int64_t gemm_launch_workspace(int engine, int M, int N, int K) {
-    if (takes_skinny(engine, 1, N, GemmEpilogue{})) return 0;
+    if (plain_auto(engine, 1, GemmEpilogue{}) && gemm_auto_kernel(M, N, K) != GEMM_KERNEL_TILES) return 0;
     GemmPlan plan;
     if (gemm_plan_from_engine(engine, M, N, K, &plan) != OK) return -1;
     return gemm_workspace_floats(plan, M, N);
@@ -605,7 +605,8 @@ std::int64_t gemm_launch_workspace(int engine, int M, int N, int K) {
 int gemm_launch(int engine, hipStream_t stream, const GemmOperands& o, const GemmEpilogue& e, float* workspace,
                 std::int64_t workspace_floats) {
     const int M = o.M, N = o.N, K = o.K;
-    if (takes_skinny(engine, o.batch, N, e)) {
+    const int kernel = plain_auto(engine, o.batch, e) ? gemm_auto_kernel(M, N, K) : GEMM_KERNEL_TILES;
+    if (kernel == GEMM_KERNEL_SKINNY) {
         GemmParams p = epilogue_params(e, M, N, o.ldc);
         p.A = o.a;
         p.B = o.b;
@@ -617,7 +618,7 @@ int gemm_launch(int engine, hipStream_t stream, const GemmOperands& o, const Gem
         launch(gemm_skinny_kernel, blocks_for(M, 4), 256, 0, stream, p, o.trans_a ? 1 : 0, o.trans_b ? 1 : 0);
         return MFH_CHECK_LAUNCH("gemm_skinny", stream);
     }
-    if (plain_auto(engine, o.batch, e) && gemm_takes_small(M, N, K)) {
+    if (kernel == GEMM_KERNEL_SMALL) {
         GemmParams p = epilogue_params(e, M, N, o.ldc);
         p.A = o.a;
         p.B = o.b;

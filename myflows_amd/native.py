@@ -35,6 +35,7 @@ GRID_LIMIT = 65535
 # The one GEMM engine is FP32 on the matrix cores; "register" is accepted as its name too, so code
 # written against the reference's register engine runs unchanged.
 GEMM_ENGINES = {"mfma": 1, "register": 1}
+GEMM_KERNELS = ("tiles", "skinny", "small")  # the values of mfh_gemm_kernel
 MATMUL_VARIANTS = {"basic": 0, "tiled": 1, "shared": 2, "register": 4}
 MATMUL_ACCUMULATION = {"fp32": 0, "kahan": 1, "dot2": 2}
 ACTIVATION_CODES = {None: 0, "relu": 1, "leaky_relu": 2}
@@ -112,6 +113,7 @@ _SIGNATURES = {
     "mfh_gemm_tile_stages": ("i", "i"),
     "mfh_gemm_tile_groups": ("i", "i"),
     "mfh_gemm_plan": ("i", "iiiPP"),
+    "mfh_gemm_kernel": ("i", "iii"),
     "mfh_gemm_workspace": ("q", "iii"),
     "mfh_split_reduce": ("i", "pp" + "iiiii" + "p"),
     "mfh_gemm": ("i", "iiipppp" + "iiiiii" + "pqp"),
@@ -157,6 +159,12 @@ def load_library():
         except (_build.BuildError, OSError) as exc:
             raise NativeHipError(f"could not build {LIBRARY_PATH}: {exc}") from exc
     return _declare(ctypes.CDLL(str(LIBRARY_PATH)))
+
+
+@lru_cache(maxsize=1)
+def _host_library():
+    """The library for queries that need no device."""
+    return load_library()
 
 
 @lru_cache(maxsize=1)
@@ -461,8 +469,23 @@ def _engine_for(engine, layout, m, n, k):
     return engine
 
 
-def _workspace_floats(engine, m, n, k):
+@lru_cache(maxsize=2048)
+def _auto_kernel(m, n, k):
+    """The kernel of GEMM_KERNELS that engine 1 runs for an m x n dense output over k (a rule on the
+    sizes alone, the same on every device)."""
+    lib = _host_library()
+    kernel = lib.mfh_gemm_kernel(m, n, k)
+    if kernel < 0:
+        _raise_for(2, lib)
+    return GEMM_KERNELS[kernel]
+
+
+def _workspace_floats(engine, m, n, k, dense=True):
+    """Split-K workspace of one product; dense: its output is (rows x columns as they come), so that a
+    small or narrow one runs on a kernel that takes none."""
     if engine == GEMM_ENGINES["mfma"]:
+        if dense and _auto_kernel(m, n, k) != "tiles":
+            return 0
         floats = _library().mfh_gemm_workspace(m, n, k)
         if floats < 0:
             _raise_for(2, _library())
@@ -473,8 +496,8 @@ def _workspace_floats(engine, m, n, k):
 
 
 def _workspace(*problems):
-    """One float32 buffer large enough for every (engine, m, n, k) GEMM of a call (they run in
-    stream order, so they can share it); (None, 0) when none of them splits K."""
+    """One float32 buffer large enough for every (engine, m, n, k[, dense]) GEMM of a call (they run
+    in stream order, so they can share it); (None, 0) when none of them splits K."""
     floats = max((_workspace_floats(*p) for p in problems), default=0)
     if not floats:
         return None, 0
@@ -715,7 +738,7 @@ def conv2d_forward(x, weight, bias=None, *, stride=(1, 1), padding=(0, 0), activ
         engine = _engine_for(engine, "NT", g.m, g.co, g.k)
         workspace, floats = _workspace((engine, g.m, g.co, g.k))
     else:  # one GEMM W cols^T over all images, stored into NCHW
-        workspace, floats = _workspace((engine, g.co, g.m, g.k))
+        workspace, floats = _workspace((engine, g.co, g.m, g.k, False))  # y is written in segments
     _call("mfh_conv_forward", x.data_ptr(), weight.data_ptr(), _addr(bias), cols.data_ptr(), _addr(rows),
           y.data_ptr(), *g.c_args(), act, alpha, engine, _addr(workspace), floats, _stream())
     return y, cols
@@ -1049,7 +1072,8 @@ def matmul(a, b, bias=None, *, variant="shared", tile=32, accumulate="kahan", ou
 
 
 def gemm_plan(m, n, k, *, layout=None):
-    """(tile name, split-K slices) the MFMA engine picks for an m x n output over k."""
+    """(tile name, split-K slices) the MFMA engine picks for an m x n output over k, where its tiles run
+    it (gemm_kernel)."""
     if min(m, n, k) <= 0:
         raise ValueError("gemm dimensions must be positive")
     if layout is not None and os.environ.get("MFHIP_GEMM_AUTOTUNE") == "1":
@@ -1059,6 +1083,15 @@ def gemm_plan(m, n, k, *, layout=None):
     tile, slices = ctypes.c_int(), ctypes.c_int()
     _call("mfh_gemm_plan", m, n, k, ctypes.byref(tile), ctypes.byref(slices))
     return list(tile_catalog())[tile.value], slices.value
+
+
+def gemm_kernel(m, n, k):
+    """What gemm runs for an m x n output over k without an explicit (or autotuned) plan: "tiles" (the
+    plan of gemm_plan), "skinny" (at most 8 columns: a wave per output row) or "small" (one launch of
+    32 x 32 tiles whose K eight waves share, the partial tiles added in FP64 and rounded once)."""
+    if min(m, n, k) <= 0:
+        raise ValueError("gemm dimensions must be positive")
+    return _auto_kernel(m, n, k)
 
 
 def split_reduce(partials, *, reference=False):
@@ -1077,9 +1110,8 @@ def split_reduce(partials, *, reference=False):
 
 
 def gemm(a, b, bias=None, *, trans_a=False, trans_b=False, engine="mfma", out=None, plan=None):
-    """Row-major ``op(a) @ op(b) (+ bias)`` on the MFMA engine (the automatic plan of a product with
-    at most 8 output columns takes a one-wave-per-row kernel instead: lanes split K, a fixed
-    butterfly adds them).
+    """Row-major ``op(a) @ op(b) (+ bias)`` on the MFMA engine. Without a plan, narrow and small products
+    take kernels of their own beside its tiles (gemm_kernel).
 
     op(a) = a.T when trans_a (a stored K x M), op(b) = b.T when trans_b (b stored N x K); not both.
     plan=(tile, slices) forces a tile of tile_catalog() and a split-K slice count.

@@ -180,6 +180,19 @@ def test_tile_loads_read_no_byte_outside_the_operand(tmp_path):
     assert run.returncode == 0, (run.returncode, run.stdout)
 
 
+@pytest.mark.parametrize("m,n,k,kernel", (
+    (64, 8, 512, "skinny"), (64, 9, 512, "small"), (1, 9, 1, "small"), (512, 512, 1024, "small"),  # 256 tiles
+    (512, 512, 1025, "tiles"), (8224, 32, 512, "small"), (8224, 32, 513, "tiles"),  # 257
+    (32, 16384, 512, "small"), (32, 16385, 512, "tiles"), (32, 16385, 16, "tiles"),  # 512, 513
+    (4096, 4096, 4096, "tiles")))
+def test_the_kernel_of_a_product_at_the_limits_of_the_rule(m, n, k, kernel):
+    assert native.gemm_kernel(m, n, k) == kernel
+    if kernel != "tiles":  # and no split-K workspace is allocated for it
+        assert native._workspace((1, m, n, k)) == (None, 0)
+    with pytest.raises(ValueError):
+        native.gemm_kernel(m, 0, k)
+
+
 def test_tile_catalogue_and_plan_codes():
     catalogue = native.tile_catalog()
     assert catalogue["128x128"][0] == 0

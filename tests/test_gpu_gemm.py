@@ -293,11 +293,13 @@ def test_k_grouped_tile_is_the_group_order_sum_of_one_group_products(layout, m, 
 
 @pytest.mark.parametrize("layout", ("NN", "NT", "TN"))
 @pytest.mark.parametrize("m,n,k", ((1, 9, 1), (32, 32, 16), (33, 31, 17), (31, 65, 127), (64, 96, 128), (100, 130, 257),
-                                   (256, 1000, 512), (512, 1024, 129), (45, 33, 2047), (17, 40, 2048)))
+                                   (256, 1000, 512), (512, 1024, 129), (45, 33, 1023), (17, 40, 1024),
+                                   (16384, 32, 512), (32, 16384, 17)))
 def test_small_products_at_the_edges_of_their_tiles_and_runs(layout, m, n, k):
     """gemm_small.hip: 32 x 32 tiles, eight runs of K in 16-deep steps, idle and ragged runs, both load
     widths. Each output is k float32 multiply-adds in some order: |error| <= (k + 16) * 2^-24 * |A||B|."""
     print("small", layout, m, n, k, flush=True)
+    assert native.gemm_kernel(m, n, k) == "small"
     rng = np.random.default_rng(k)
     a, b = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(k, n)).astype(np.float32)
     bias = rng.normal(size=(n,)).astype(np.float32)
@@ -317,6 +319,7 @@ def test_small_products_add_their_runs_of_k_in_fp64(layout, m, n, k):
     ranges, added in run order in FP64 and rounded once, as a split plan's slices are; the bias is added
     after the rounding. Bit for bit."""
     print("small runs", layout, m, n, k, flush=True)
+    assert native.gemm_kernel(m, n, k) == "small"
     trans_a, trans_b = LAYOUTS[layout]
     rng = np.random.default_rng(9)
     a, b, _, _ = operands(rng, m, n, k, trans_a, trans_b)
@@ -328,6 +331,24 @@ def test_small_products_add_their_runs_of_k_in_fp64(layout, m, n, k):
     expected = gpu(fp64_slice_sum(np.stack([host(part) for part in parts])))
     assert torch.equal(native.gemm(a, b, trans_a=trans_a, trans_b=trans_b), expected)
     assert torch.equal(native.gemm(a, b, bias, trans_a=trans_a, trans_b=trans_b), expected + bias)
+
+
+@pytest.mark.parametrize("m,n,k,kernel", ((512, 512, 1024, "small"), (512, 512, 1025, "tiles"), (8224, 32, 512, "small"),
+                                          (8224, 32, 513, "tiles"), (32, 16384, 64, "small"), (32, 16385, 64, "tiles"),
+                                          (64, 9, 100, "small"), (64, 8, 100, "skinny")))
+def test_the_named_kernel_is_the_one_that_runs(m, n, k, kernel):
+    """native.gemm_kernel at the limits of its rule, by bits: "tiles" are those of gemm_plan's plan, "small"
+    those of the runs' FP64 sum, which the tiles' one float32 chain, or split, does not give."""
+    print("kernel", m, n, k, kernel, flush=True)
+    assert native.gemm_kernel(m, n, k) == kernel
+    rng = np.random.default_rng(10)
+    a, b = gpu(rng.standard_normal((m, k)).astype(np.float32)), gpu(rng.standard_normal((k, n)).astype(np.float32))
+    got = native.gemm(a, b)
+    assert torch.equal(got, native.gemm(a, b, plan=native.gemm_plan(m, n, k))) == (kernel == "tiles")
+    run = -(-(-(-k // 8)) // 16) * 16
+    parts = [native.gemm(a[:, lo:lo + run].contiguous(), b[lo:lo + run].contiguous(), plan=("64x64", 1))
+             for lo in range(0, k, run)]
+    assert torch.equal(got, gpu(fp64_slice_sum(np.stack([host(p) for p in parts])))) == (kernel == "small")
 
 
 def test_small_products_keep_infinities_to_their_own_rows_and_columns():
