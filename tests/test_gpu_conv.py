@@ -327,6 +327,26 @@ def test_rows_path_forward_matches_the_nchw_gemm(case, monkeypatch):
     assert_near(host(rows), np.maximum(pre, 0), 1e-5, "rows")
 
 
+@pytest.mark.parametrize("n,ci,co,h,w", ((3, 5, 24, 9, 11), (2, 3, 7, 5, 6)))
+def test_small_column_gradients_are_exact(n, ci, co, h, w):
+    """dX of the im2col algorithm through a gated dy: the column gradient W^T dy^T over all pixels, the only
+    product with both operands transposed, on the small-product kernel. Whole numbers: exact."""
+    rng = np.random.default_rng(n + co)
+    x, weight = rng.integers(-3, 4, (n, ci, h, w)), rng.integers(-3, 4, (co, ci, 3, 3))
+    grad = rng.integers(-3, 4, (n, co, (h - 1) // 2 + 1, (w - 1) // 2 + 1))
+    pixels = n * grad.shape[2] * grad.shape[3]
+    print("small column gradient", (ci * 9, pixels, co), flush=True)
+    assert native.gemm_kernel(ci * 9, pixels, co) == "small"
+    output = rng.integers(0, 2, grad.shape).astype(np.float32)  # the gate: where the forward output is positive
+    dx, _, _ = native.conv2d_backward(gpu(x.astype(np.float32)), gpu(weight.astype(np.float32)),
+                                      gpu(grad.astype(np.float32)), None, stride=(2, 2), padding=(1, 1),
+                                      need_bias_grad=False, need_weight_grad=False, activation="relu",
+                                      output=gpu(output), algorithm="im2col", recompute_cols=True)
+    exact = torch.nn.grad.conv2d_input((n, ci, h, w), torch.as_tensor(weight, dtype=torch.float64),
+                                       torch.as_tensor(grad * output, dtype=torch.float64), stride=2, padding=1)
+    np.testing.assert_array_equal(host(dx), exact.numpy().astype(np.float32))
+
+
 def permuted_kernel(w, flip):
     """The kernel in the order an implicit product reads it, by plain tensor permutes: rows co over
     features (ci, tap) (flip 0), or rows ci over (co, KH*KW-1-tap) (flip 1); a multiple of 32

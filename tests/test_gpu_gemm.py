@@ -107,8 +107,9 @@ def test_misaligned_operands_take_the_scalar_loads():
             db = torch.empty(b.size + 1, device="cuda")[1:].view(b.shape)
             da.copy_(gpu(a))
             db.copy_(gpu(b))
-            got = host(native.gemm(da, db, trans_a=trans_a, trans_b=trans_b)).astype(np.float64)
-            assert np.all(np.abs(got - exact) <= gamma_k(k) * magnitude + 1e-30)
+            for plan in (None, ("64x64", 1), ("64x64k2", 1)):  # the small products' loads and the tiles'
+                got = host(native.gemm(da, db, trans_a=trans_a, trans_b=trans_b, plan=plan)).astype(np.float64)
+                assert np.all(np.abs(got - exact) <= gamma_k(k) * magnitude + 1e-30)
 
 
 def test_split_k_plan_workspace_and_accuracy():
