@@ -449,7 +449,7 @@ def c2_gemms(reps=20):
         us = _event_time_us(lambda: native.gemm(a, b, trans_a=trans_a, out=c), reps=reps)
         tflops = 2.0 * m * n * k / (us * 1e-6) / 1e12
         tile, slices = native.gemm_plan(m, n, k, layout="TN" if trans_a else "NN")
-        kernel = native.gemm_kernel(m, n, k)
+        kernel = native.gemm_kernel(m, n, k, layout="TN" if trans_a else "NN")
         out[name] = {"us": round(us, 2), "TFLOP/s": round(tflops, 2), "frac": round(tflops / FP32_MFMA_PEAK_TFLOPS, 3),
                      "plan": f"tile {tile} slices {slices}" if kernel == "tiles" else f"gemm_{kernel}_kernel"}
         del a, b, c

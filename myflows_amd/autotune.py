@@ -1,6 +1,7 @@
 """Opt-in empirical GEMM plans (MFHIP_GEMM_AUTOTUNE=1): for each (layout, M, N, K) the MFMA
-engine's tiles and split-K counts are timed on this device and the fastest is kept, in a JSON file
-per shape under MFHIP_AUTOTUNE_CACHE (default: ``myflows_amd/_gemm_plans``). The reference's
+engine's tiles and split-K counts are timed on this device and the fastest is kept; where the
+automatic choice is a kernel beside the tiles (native.gemm_kernel: narrow and small products) that
+kernel is timed too, and stays the choice when no tile plan beats it. One JSON file per shape under MFHIP_AUTOTUNE_CACHE (default: ``myflows_amd/_gemm_plans``). The reference's
 ``ops/cuda_native/autotune.py:1-195`` plays the same role for its register engine.
 
 Each measurement writes ``{"identity", "layout", "shape", "candidates", "selected"}``. A file is
@@ -27,7 +28,7 @@ import torch
 
 from . import native
 
-VERSION = 1
+VERSION = 2
 SPLIT_CHOICES = (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64)
 LAYOUTS = ("NN", "NT", "TN")
 
@@ -57,15 +58,26 @@ def plan_file(layout, m, n, k, device_index=None):
 
 def read_plan(path, layout, shape, identity):
     """(tile, requested slices) from a stored measurement, or None if it is missing or stale."""
+    found = _read(path, layout, shape, identity)
+    return found[:2] if found else None
+
+
+def _read(path, layout, shape, identity):
+    """(tile, requested slices, whether the automatic kernel beat them) or None."""
     try:
         record = json.loads(Path(path).read_text(encoding="utf-8"))
         if record["identity"] != identity or record["layout"] != layout or record["shape"] != list(shape):
             return None
         tile, requested = record["selected"]["tile"], record["selected"]["requested_slices"]
         native._plan_code(tile, requested)  # still a valid plan of this library
-        return tile, requested
+        return tile, requested, _automatic_wins(record)
     except (OSError, ValueError, KeyError, TypeError):
         return None
+
+
+def _automatic_wins(record):
+    median = record.get("automatic", {}).get("median_ms")
+    return median is not None and median <= record["selected"]["median_ms"]
 
 
 def write_plan(path, record):
@@ -104,18 +116,30 @@ def candidates(m, n, k, workspace_budget_bytes):
 
 
 def measure(layout, m, n, k, repeats=3, rounds=3, seed=197):
-    """Time every candidate plan of one GEMM shape; returns the record that write_plan stores."""
+    """Time every candidate plan of one GEMM shape, and the automatic kernel where it is none of them;
+    returns the record that write_plan stores ("selected" is the fastest tile plan)."""
     trans_a, trans_b = layout == "TN", layout == "NT"
     gen = torch.Generator(device="cuda").manual_seed(seed)
     a = torch.randn((k, m) if trans_a else (m, k), device="cuda", generator=gen)
     b = torch.randn((n, k) if trans_b else (k, n), device="cuda", generator=gen)
     out = torch.empty((m, n), device="cuda")
+    ahead = torch.zeros(1 << 26, device="cuda")  # a pass over it (about 0.1 ms) keeps the GPU busy while
+    # the host issues a timing's launches: products shorter than a launch's issue would all time alike
     free, total = torch.cuda.mem_get_info()
     budget = max(0, int(free) - max(512 << 20, int(total) // 8))
     rows = [{"tile": t, "requested_slices": r, "slices": s, "workspace_bytes": w, "times_ms": []}
             for t, r, s, w in candidates(m, n, k, budget)]
-    launch = lambda row: native.gemm(a, b, trans_a=trans_a, trans_b=trans_b, out=out,
-                                     plan=(row["tile"], row["requested_slices"]))
+    auto_tile, auto_slices = native.gemm_plan(m, n, k)
+    automatic = {"tile": auto_tile, "slices": auto_slices, "kernel": native.gemm_kernel(m, n, k)}
+    code = lambda row: (native.GEMM_ENGINES["mfma"] if row is automatic
+                        else native._plan_code(row["tile"], row["requested_slices"]))
+
+    def launch(row):
+        engine = code(row)
+        workspace, floats = native._workspace((engine, m, n, k))
+        native._call("mfh_gemm", engine, int(trans_a), int(trans_b), a.data_ptr(), b.data_ptr(), 0, out.data_ptr(), m,
+                     n, k, int(a.shape[1]), int(b.shape[1]), n, native._addr(workspace), floats, native._stream())
+
     reference_bits = {}
     for row in rows:  # correctness pass: the unsplit tiles of one K-group count must give the same bits
         launch(row)
@@ -128,42 +152,57 @@ def measure(layout, m, n, k, repeats=3, rounds=3, seed=197):
     start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     order = random.Random(2201)
     began = time.monotonic()
+    timed = list(rows)
+    if automatic["kernel"] != "tiles":
+        automatic["times_ms"] = []
+        timed.append(automatic)
+        launch(automatic)
     for _ in range(rounds):
-        order.shuffle(rows)
-        for row in rows:
+        order.shuffle(timed)
+        for row in timed:
+            ahead.add_(1.0)
             start.record()
             for _ in range(repeats):
                 launch(row)
             stop.record()
             stop.synchronize()
             row["times_ms"].append(start.elapsed_time(stop) / repeats)
-    for row in rows:
+    for row in timed:
         row["median_ms"] = statistics.median(row["times_ms"])
     best = min(rows, key=lambda row: row["median_ms"])
-    auto_tile, auto_slices = native.gemm_plan(m, n, k)
     _, identity = device_identity(torch.cuda.current_device())
     return {"identity": identity, "layout": layout, "shape": [m, n, k], "candidates": rows, "selected": best,
-            "automatic": {"tile": auto_tile, "slices": auto_slices}, "seconds": time.monotonic() - began}
+            "automatic": automatic, "seconds": time.monotonic() - began}
 
 
 @lru_cache(maxsize=4096)
 def _selected(root, device_index, layout, m, n, k):
     path = plan_file(layout, m, n, k, device_index)
     _, identity = device_identity(device_index)
-    found = read_plan(path, layout, (m, n, k), identity)
+    found = _read(path, layout, (m, n, k), identity)
     if found:
         return found
     with _locked(path.parent):
-        found = read_plan(path, layout, (m, n, k), identity)  # another process may have measured it
+        found = _read(path, layout, (m, n, k), identity)  # another process may have measured it
         if found:
             return found
         record = measure(layout, m, n, k)
         write_plan(path, record)
-        return record["selected"]["tile"], record["selected"]["requested_slices"]
+        return record["selected"]["tile"], record["selected"]["requested_slices"], _automatic_wins(record)
 
 
 def selected_plan(layout, m, n, k):
-    """(tile name, requested split count) for an op(A) op(B) GEMM of this shape on this device."""
+    """(tile name, requested split count) of the fastest tile plan for an op(A) op(B) GEMM of this shape
+    on this device."""
+    return _choice(layout, m, n, k)[:2]
+
+
+def prefers_automatic(layout, m, n, k):
+    """Whether the automatic kernel beside the tiles was measured no slower than that plan."""
+    return _choice(layout, m, n, k)[2]
+
+
+def _choice(layout, m, n, k):
     if layout not in LAYOUTS or min(m, n, k) < 1:
         raise ValueError("expected layout NN, NT or TN and positive GEMM dimensions")
     return _selected(str(cache_root()), torch.cuda.current_device(), layout, int(m), int(n), int(k))

@@ -462,11 +462,19 @@ def _explicit_split(code):
 
 
 def _engine_for(engine, layout, m, n, k):
-    """The automatic engine, or the autotuned plan when MFHIP_GEMM_AUTOTUNE=1."""
-    if engine == GEMM_ENGINES["mfma"] and os.environ.get("MFHIP_GEMM_AUTOTUNE") == "1":
+    """The automatic engine, or the autotuned plan of a dense product when MFHIP_GEMM_AUTOTUNE=1."""
+    if engine == GEMM_ENGINES["mfma"] and _autotuned(layout, m, n, k):
         from .autotune import selected_plan
         return _plan_code(*selected_plan(layout, m, n, k))
     return engine
+
+
+def _autotuned(layout, m, n, k):
+    """Whether MFHIP_GEMM_AUTOTUNE=1 and a tile plan was measured faster than the automatic kernel."""
+    if os.environ.get("MFHIP_GEMM_AUTOTUNE") != "1":
+        return False
+    from .autotune import prefers_automatic
+    return not prefers_automatic(layout, m, n, k)
 
 
 @lru_cache(maxsize=2048)
@@ -1076,7 +1084,7 @@ def gemm_plan(m, n, k, *, layout=None):
     it (gemm_kernel)."""
     if min(m, n, k) <= 0:
         raise ValueError("gemm dimensions must be positive")
-    if layout is not None and os.environ.get("MFHIP_GEMM_AUTOTUNE") == "1":
+    if layout is not None and _autotuned(layout, m, n, k):
         from .autotune import selected_plan
         tile, requested = selected_plan(layout, m, n, k)
         return tile, _slices(k, requested, tile_catalog()[tile][-1])
@@ -1085,13 +1093,14 @@ def gemm_plan(m, n, k, *, layout=None):
     return list(tile_catalog())[tile.value], slices.value
 
 
-def gemm_kernel(m, n, k):
-    """What gemm runs for an m x n output over k without an explicit (or autotuned) plan: "tiles" (the
+def gemm_kernel(m, n, k, *, layout=None):
+    """What gemm runs for an m x n output over k without an explicit plan (with a layout: or an autotuned
+    one, as gemm_plan): "tiles" (the
     plan of gemm_plan), "skinny" (at most 8 columns: a wave per output row) or "small" (one launch of
     32 x 32 tiles whose K eight waves share, the partial tiles added in FP64 and rounded once)."""
     if min(m, n, k) <= 0:
         raise ValueError("gemm dimensions must be positive")
-    return _auto_kernel(m, n, k)
+    return "tiles" if layout is not None and _autotuned(layout, m, n, k) else _auto_kernel(m, n, k)
 
 
 def split_reduce(partials, *, reference=False):

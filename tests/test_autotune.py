@@ -26,6 +26,23 @@ def test_plan_record_round_trip_and_stale_records(tmp_path):
     assert autotune.read_plan(path, "TN", (64, 576, 72384), identity) is None
 
 
+def test_a_record_may_prefer_the_automatic_kernel(tmp_path):
+    identity = {"cus": 256}
+    record = {"identity": identity, "layout": "NN", "shape": [100, 130, 257], "candidates": [],
+              "selected": {"tile": "64x64", "requested_slices": 2, "median_ms": 0.009},
+              "automatic": {"tile": "64x64", "slices": 1, "kernel": "small", "median_ms": 0.006}}
+    path = tmp_path / "NN-100x130x257.json"
+    read = lambda: autotune._read(path, "NN", (100, 130, 257), identity)
+    autotune.write_plan(path, record)
+    assert read() == ("64x64", 2, True)
+    record["automatic"]["median_ms"] = 0.010
+    autotune.write_plan(path, record)
+    assert read() == ("64x64", 2, False)
+    del record["automatic"]["median_ms"]  # the automatic choice was a tile plan, one of the candidates
+    autotune.write_plan(path, record)
+    assert read() == ("64x64", 2, False)
+
+
 def test_candidates_are_distinct_and_within_budget():
     rows = autotune.candidates(64, 576, 72384, workspace_budget_bytes=64 << 20)
     assert rows and all(w <= 64 << 20 for *_, w in rows)
@@ -49,3 +66,24 @@ def test_measured_plan_is_stored_and_used(tmp_path, monkeypatch):
     tuned = native.gemm(a, b, trans_a=True)
     explicit = native.gemm(a, b, trans_a=True, plan=(tile, requested))
     assert torch.equal(tuned, explicit)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", ((512, 512, 512), (100, 130, 1001)))
+def test_small_products_are_measured_against_their_own_kernel(tmp_path, monkeypatch, m, n, k):
+    """The automatic kernel of a product that is not on the tiles is timed beside the tile plans, and the
+    product keeps it unless one of them is faster."""
+    print("autotune", m, n, k, flush=True)
+    monkeypatch.setenv("MFHIP_AUTOTUNE_CACHE", str(tmp_path))
+    monkeypatch.setenv("MFHIP_GEMM_AUTOTUNE", "1")
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    a, b = torch.randn((m, k), device="cuda", generator=gen), torch.randn((k, n), device="cuda", generator=gen)
+    tuned = native.gemm(a, b)
+    record = json.loads(autotune.plan_file("NN", m, n, k).read_text())
+    print({key: record[key]["median_ms"] for key in ("automatic", "selected")}, flush=True)
+    assert record["automatic"]["kernel"] == "small" and len(record["automatic"]["times_ms"]) > 0
+    wins = record["automatic"]["median_ms"] <= record["selected"]["median_ms"]
+    assert autotune.prefers_automatic("NN", m, n, k) == wins
+    assert native.gemm_kernel(m, n, k, layout="NN") == ("small" if wins else "tiles")
+    monkeypatch.delenv("MFHIP_GEMM_AUTOTUNE")
+    assert torch.equal(tuned, native.gemm(a, b)) == wins
