@@ -19,12 +19,12 @@ namespace mfh {
 namespace {
 
 constexpr int HEAD_THREADS = 256;
-constexpr int LOSS_THREADS = 1024;  // one workgroup forms the loss
+constexpr int LOSS_THREADS = 1024;  // of a workgroup of the loss
 
 // LANES lanes share a plane: lane l adds elements l, l + LANES, ... in FP64 (four loads in flight),
 // then a fixed butterfly adds the lanes. One thread per plane read a cache line per lane and element
-// and left all but planes / 64 waves idle: 64 x 64 planes of 29 x 39 took 324 us for 18.5 MB
-// (the stem's whole training pass went from 677 to 336 us with the lanes below).
+// and left all but planes / 64 waves idle: 64 x 64 planes of 29 x 39 took 327 us for 18.5 MB in a
+// training pass, with 64 lanes 5.1.
 template <int LANES>
 __global__ __launch_bounds__(HEAD_THREADS) void plane_mean_kernel(const float* __restrict__ x, float* __restrict__ y,
                                                                   long long planes, int hw) {
@@ -57,12 +57,16 @@ __global__ __launch_bounds__(HEAD_THREADS) void plane_mean_backward_kernel(const
     dx[i] = add ? dx[i] + v : v;
 }
 
-// The squared differences of 256 x 1000 outputs took one workgroup 70 us, a load at a time; a CU's own
-// bandwidth bounds it, so larger counts take several workgroups. The sums are formed by LOSS_THREADS-thread workgroups: thread t of the grid adds
-// those of elements t, t + threads, ... in that order in FP64 with LOSS_AHEAD loads of each operand
-// in flight; a workgroup's thread sums are combined by a fixed tree in LDS. A single workgroup
-// writes the loss; several write their sums to partials, which mse_finish_kernel adds.
+// Thread t of the grid adds the squares of elements t, t + threads, ... in that order in FP64, with
+// LOSS_AHEAD loads of each operand in flight; a workgroup's thread sums are combined by a fixed tree in
+// LDS. A single workgroup writes the loss; several write their sums to partials, which mse_finish_kernel
+// adds. One workgroup with a load in flight took 70 us for 256 x 1000 elements in a training pass, a
+// CU's own latency and bandwidth bounding it; 32 workgroups take 5.1 and the finish 2.7.
 constexpr int LOSS_AHEAD = 8;
+// A fixed cap, so that the order of the sum does not depend on the device; the finish reads one partial
+// a thread.
+constexpr int LOSS_GROUPS_MAX = 256;
+static_assert(LOSS_GROUPS_MAX <= LOSS_THREADS, "mse_finish_kernel reads one partial per thread");
 
 __device__ __forceinline__ double tree_sum(double* partial, double s) {
     partial[threadIdx.x] = s;
@@ -113,7 +117,7 @@ __global__ __launch_bounds__(LOSS_THREADS) void mse_loss_kernel(const float* __r
     else loss[0] = mean_of(sum, count);
 }
 
-// The workgroups' sums (at most LOSS_THREADS), added by the same tree.
+// The workgroups' sums (at most LOSS_GROUPS_MAX), added by the same tree.
 __global__ __launch_bounds__(LOSS_THREADS) void mse_finish_kernel(const double* __restrict__ partials, int groups,
                                                                   float* __restrict__ loss, long long count) {
     __shared__ double partial[LOSS_THREADS];
@@ -171,7 +175,9 @@ __global__ __launch_bounds__(SPAN* GROUPS) void column_sums_kernel(const float* 
 int launch_plane_mean(const float* x, float* y, std::int64_t planes, int hw, hipStream_t stream) {
     if (planes == 0) return OK;
     // A wave per plane from two full passes of it on; 16 lanes for the small planes of a network's end
-    // (4 x 5, 7 x 7), of which a wave then takes four; one thread where 16 lanes would mostly idle.
+    // (4 x 5, 7 x 7), of which a wave then takes four; one thread where 16 lanes would mostly idle. us for
+    // 4096 planes by one thread each / as here: of 16 elements 3.4 / 2.1, of 49 7.5 / 2.4, of 127 17.4 /
+    // 2.5, of 128 16.2 / 2.7, of 1131 148 / 4.1; for 32768 of 128, 17.0 / 6.9 (of 127 by 16 lanes 3.8).
     const auto run = [&](auto kernel, int lanes) {
         launch(kernel, blocks_for(planes * lanes, HEAD_THREADS), HEAD_THREADS, 0, stream, x, y, planes, hw);
     };
@@ -189,11 +195,12 @@ int launch_plane_mean_backward(const float* dy, float* dx, std::int64_t planes, 
     return MFH_CHECK_LAUNCH("plane_mean_backward", stream);
 }
 
-// Workgroups of the loss of count elements: one while its loads are a few rounds (a second launch
-// costs about 3 us), else one per LOSS_AHEAD rounds up to the device's CUs.
+// Workgroups of the loss of count elements: one while its loads are a few rounds (32768 elements 4.3 us,
+// 6.0 before its loads were LOSS_AHEAD deep), as the finish is a second launch, else one per LOSS_AHEAD
+// rounds up to LOSS_GROUPS_MAX (32769 elements 5.6 us, 65536 5.4 where one workgroup took 9.8).
 int mse_loss_groups(std::int64_t count) {
     if (count <= 4LL * LOSS_AHEAD * LOSS_THREADS) return 1;
-    return static_cast<int>(std::min<std::int64_t>(256, blocks_for(count, LOSS_AHEAD * LOSS_THREADS)));
+    return static_cast<int>(std::min<std::int64_t>(LOSS_GROUPS_MAX, blocks_for(count, LOSS_AHEAD * LOSS_THREADS)));
 }
 
 int launch_mse_loss(const float* pred, const float* target, float* loss, std::int64_t count, double* partials,
