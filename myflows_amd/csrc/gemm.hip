@@ -39,6 +39,30 @@ constexpr int NAMED_TILE_OF[NAMED_COUNT] = {0, 1, 4, 2, 5};
 // output's K terms in one order.
 constexpr int GEMM_PAIR = 8;
 
+// The global reads of one stage of both operands: the quads of both, then what is left to read singly of
+// both. In one place, the single floats wait for the quads in flight once; after each operand's quads they
+// waited twice in the last stage (1531 x 1000 over 777, B transposed, 38.7 -> 36.9 us in a loop of calls).
+template <bool TA, bool TB, class LoadA, class LoadB>
+__device__ __forceinline__ void fetch_operands(LoadA& la, LoadB& lb, const GemmParams& p, const float* __restrict__ A,
+                                               const float* __restrict__ B, int m0, int n0, int kt, int k_end,
+                                               int tid) {
+    bool a, b;
+    if constexpr (TA) a = la.load_quads(A, p.lda, kt, k_end, m0, p.M, tid);
+    else a = la.load_quads(A, p.lda, m0, p.M, kt, k_end, tid);
+    if constexpr (TB) b = lb.load_quads(B, p.ldb, n0, p.N, kt, k_end, tid);
+    else b = lb.load_quads(B, p.ldb, kt, k_end, n0, p.N, tid);
+    if (a || b) {
+        if (a) {
+            if constexpr (TA) la.load_singles(A, p.lda, kt, k_end, m0, p.M, tid);
+            else la.load_singles(A, p.lda, m0, p.M, kt, k_end, tid);
+        }
+        if (b) {
+            if constexpr (TB) lb.load_singles(B, p.ldb, n0, p.N, kt, k_end, tid);
+            else lb.load_singles(B, p.ldb, kt, k_end, n0, p.N, tid);
+        }
+    }
+}
+
 template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VA, bool VB>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma_kernel(GemmParams p) {
     using S = MfmaShape<BM, BN, BK, WM, WN, TA, TB, 4, 4, GEMM_PAIR>;
@@ -54,17 +78,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma_kernel(G
     float* __restrict__ C = p.C + z * p.c_batch;
     const int k_begin = p.split ? z * p.k_chunk : 0;
     const int k_end = p.split ? min(p.K, k_begin + p.k_chunk) : p.K;
-    const int M = p.M, N = p.N;
 
     // A tile: rows = m (k-contiguous) or k (mn-contiguous); likewise B.
     TileLoader<TA ? BK : BM, TA ? BM : BK, S::THREADS, VA, TA> la;
     TileLoader<TB ? BN : BK, TB ? BK : BN, S::THREADS, VB, !TB> lb;
-    auto fetch = [&](int kt) {
-        if constexpr (TA) la.load(A, p.lda, kt, k_end, m0, M, tid);
-        else la.load(A, p.lda, m0, M, kt, k_end, tid);
-        if constexpr (TB) lb.load(B, p.ldb, n0, N, kt, k_end, tid);
-        else lb.load(B, p.ldb, kt, k_end, n0, N, tid);
-    };
+    auto fetch = [&](int kt) { fetch_operands<TA, TB>(la, lb, p, A, B, m0, n0, kt, k_end, tid); };
     auto store = [&](float* a_lds, float* b_lds) {
         la.template store<S::LDA_S>(a_lds, tid);
         lb.template store<S::LDB_S>(b_lds, tid);
@@ -97,7 +115,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_grouped_
 
     int tile_m, tile_n, z;
     tile_of_workgroup(tile_m, tile_n, z);
-    const int group = threadIdx.x / S::THREADS, tid = threadIdx.x % S::THREADS;
+    // The group is the same for a wave: told so, the compiler checks the edges of unaligned operands once a
+    // wave (3001 x 129 over 513 18.8 -> 18.1 us). Aligned ones have no such checks, and 1024^3 was 2 %
+    // faster with it in one layout and 2 % slower in another.
+    const int thread_group = threadIdx.x / S::THREADS, tid = threadIdx.x % S::THREADS;
+    const int group = VA && VB ? thread_group : __builtin_amdgcn_readfirstlane(thread_group);
     const int wave = tid / 64, lane = tid % 64;
     const int wm0 = (wave / S::WGN) * WM, wn0 = (wave % S::WGN) * WN;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
@@ -106,7 +128,6 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_grouped_
     float* __restrict__ C = p.C + z * p.c_batch;
     const int k_begin = p.split ? z * p.k_chunk : 0;
     const int k_end = p.split ? min(p.K, k_begin + p.k_chunk) : p.K;
-    const int M = p.M, N = p.N;
     const int per = ((k_end - k_begin + BK - 1) / BK + KG - 1) / KG;  // stages of every group
     const int g_begin = k_begin + group * per * BK;
 
@@ -115,18 +136,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_grouped_
     LoadA la[2];
     LoadB lb[2];
     // Every load is bounded by k_end (reads past it give zeros), the ahead loop's fetches past the
-    // end included. An unaligned A beside an aligned B is read second: read first, the compiler copies
-    // its quads to other registers, which waits for them a stage too early (3001 x 128 over 513 18.3 -> 17.1 us).
+    // end included.
     auto fetch = [&](auto slot, int kt) {
         constexpr int T = decltype(slot)::value;
-        const auto load_a = [&] {
-            if constexpr (TA) la[T].load(A, p.lda, kt, k_end, m0, M, tid);
-            else la[T].load(A, p.lda, m0, M, kt, k_end, tid);
-        };
-        if constexpr (VA || !VB) load_a();
-        if constexpr (TB) lb[T].load(B, p.ldb, n0, N, kt, k_end, tid);
-        else lb[T].load(B, p.ldb, kt, k_end, n0, N, tid);
-        if constexpr (!VA && VB) load_a();
+        fetch_operands<TA, TB>(la[T], lb[T], p, A, B, m0, n0, kt, k_end, tid);
     };
     auto store = [&](auto slot, float* a_lds, float* b_lds) {
         constexpr int T = decltype(slot)::value;
@@ -179,7 +192,9 @@ __device__ __forceinline__ void finish_output(const GemmParams& p, float* C, int
 
 // Row and column of output i by the multiply-and-shift division of columns = FastDiv(N) (a product
 // has at most INDEX_LIMIT outputs, so i fits an int). A 64-bit division and remainder per output
-// are some 200 vector instructions, which bounded the reductions.
+// are some 200 vector instructions: with one division a quad, four slices of 512 x 4608 outputs took
+// 27.6 us instead of 29.3 in a training pass (the slices' reads bound them), the grouped reduction of a
+// strided convolution's 24 slices of 160 x 864 5.0 instead of 6.1.
 __device__ __forceinline__ void finish_output(const GemmParams& p, const FastDiv& columns, float* C, long long i,
                                               double s) {
     int col;

@@ -20,8 +20,8 @@ typedef float UnalignedQuad __attribute__((ext_vector_type(4), aligned(4)));
 // around the quads they cost every stage of every tile: whichever of the two the compiler places second
 // waits for all loads in flight before it fills the same registers.
 // us a product on MI355X, single floats everywhere / in such a branch / as here: A^T B 1000 x 1001 over
-// 3000 77.9 / 93.0 / 71.9, 2047 x 2047 over 1023 103.6 / 113.1 / 90.4, 3001 x 129 over 513 20.2 / 25.0 /
-// 18.6; A B^T 1531 x 1000 over 777 42.6 / 39.1 / 39.5.
+// 3000 78.7 / 93.1 / 72.8, 2047 x 2047 over 1023 104.8 / 113.3 / 89.6, 3001 x 129 over 513 20.2 / 24.9 /
+// 17.9; A B^T 1531 x 1000 over 777 42.7 / 39.0 / 38.9.
 template <int ROWS, int COLS, int THREADS, bool VEC, bool ROWS_K>
 struct TileLoader {
     static constexpr int ELEMS = ROWS * COLS / 4;
@@ -30,8 +30,9 @@ struct TileLoader {
     static_assert(COLS % 4 == 0 && THREADS % VCOLS == 0, "whole quads per row, one column per thread");
     float4 v[PER_THREAD];
 
-    __device__ __forceinline__ void load(const float* __restrict__ base, int ld, int row0, int row_limit, int col0,
-                                          int col_limit, int tid) {
+    // Reads the quads; true where this lane's floats are left for load_singles (same arguments).
+    __device__ __forceinline__ bool load_quads(const float* __restrict__ base, int ld, int row0, int row_limit,
+                                                int col0, int col_limit, int tid) {
         const int col = col0 + (tid % VCOLS) * 4;
         // Whether the tile has no quad to read singly. A quad that spills over ends at most three floats
         // past its row, and a row holds one at least: with four more rows there is always enough.
@@ -53,20 +54,28 @@ struct TileLoader {
             }
             v[i] = value;
         }
-        if constexpr (!VEC) {
-            if (!whole && !quad && col < col_limit) {
+        return !whole && !quad && col < col_limit;
+    }
+
+    __device__ __forceinline__ void load_singles(const float* __restrict__ base, int ld, int row0, int row_limit,
+                                                  int col0, int col_limit, int tid) {
+        const int col = col0 + (tid % VCOLS) * 4;
 #pragma unroll
-                for (int i = 0; i < PER_THREAD; ++i) {
-                    const int f = tid + i * THREADS, row = row0 + f / VCOLS;
-                    const float* at = base + static_cast<long long>(row) * ld + col;
-                    float e[3] = {0.f, 0.f, 0.f};
+        for (int i = 0; i < PER_THREAD; ++i) {
+            const int f = tid + i * THREADS, row = row0 + f / VCOLS;
+            const float* at = base + static_cast<long long>(row) * ld + col;
+            float e[3] = {0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int u = 0; u < 3; ++u)
-                        if (f < ELEMS && row < row_limit && u < col_limit - col) e[u] = at[u];
-                    v[i] = make_float4(e[0], e[1], e[2], 0.f);
-                }
-            }
+            for (int u = 0; u < 3; ++u)
+                if (f < ELEMS && row < row_limit && u < col_limit - col) e[u] = at[u];
+            v[i] = make_float4(e[0], e[1], e[2], 0.f);
         }
+    }
+
+    __device__ __forceinline__ void load(const float* __restrict__ base, int ld, int row0, int row_limit, int col0,
+                                          int col_limit, int tid) {
+        if (load_quads(base, ld, row0, row_limit, col0, col_limit, tid))
+            load_singles(base, ld, row0, row_limit, col0, col_limit, tid);
     }
 
     template <int LD>
