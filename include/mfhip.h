@@ -481,7 +481,8 @@ MFH_API int mfh_mse_loss(uint64_t pred, uint64_t target, uint64_t loss, int64_t 
  * workgroups (0: one workgroup is enough, use mfh_mse_loss; -1: count out of range). */
 MFH_API int64_t mfh_mse_loss_workspace(int64_t count);
 
-/* mfh_mse_loss over several workgroups, whose FP64 sums (in `workspace`) a second launch adds. */
+/* mfh_mse_loss over several workgroups, whose FP64 sums (in `workspace`, 8-byte aligned and kept until both
+ * launches have run) a second launch adds. */
 MFH_API int mfh_mse_loss_split(uint64_t pred, uint64_t target, uint64_t loss, int64_t count, uint64_t workspace,
                                int64_t workspace_doubles, uint64_t stream);
 

@@ -3,7 +3,7 @@
 //
 // What bounds these products is latency, not the matrix cores: the LDS tiles of gemm.hip walk K in
 // 16-deep stages with a barrier each, and a 100 x 130 output over K = 257 is six 64 x 64 tiles of
-// nine stages, about 1 us a stage. Here a wave reads its operands straight into the MFMA's lanes
+// nine stages (two groups of waves share them), 13.1 us against 6.6 here. Here a wave reads its operands straight into the MFMA's lanes
 // (no LDS, no barrier, two 16-deep steps in flight), K is shared by eight waves of the same
 // workgroup, and the eight partial tiles are added through LDS in wave order in FP64 and rounded
 // once (the automatic plan split many of these products, and its slices are summed so): one launch,
@@ -112,12 +112,14 @@ __global__ __launch_bounds__(SMALL_THREADS) void gemm_small_kernel(GemmParams p)
 
 }  // namespace
 
-// Where one launch of these tiles is the faster one (us a call, against gemm.hip's automatic plan, of
-// which about 8.5 are the host's): 100 x 130 over K = 257 9.1 / 13.0, over 1001 10.9 / 18.6, 256 x 1000
-// over 512 9.0 / 16.0, 500 x 500 over 1001 11.8 / 18.2, 512 x 1000 over 512 11.9 / 15.8. Beyond, a
-// wave's serial run of K and the operands' traffic (each 32 x 32 tile reads its rows and columns
-// again) cost more than the tiles: 128 x 128 over 2048 16.6 / 14.1 (split K), 700 x 700 with a
-// transposed A over 1024 27.4 / 22.5.
+// Where one launch of these tiles is the faster one (us on the GPU, gemm.hip's automatic plan / here, the
+// slowest of the layouts): 64 x 10 over 16 6.2 / 4.2, 100 x 130 over 257 13.1 / 6.6, over 1000 17.8 /
+// 11.3, 256 x 1000 over 512 17.3 / 8.0, 500 x 500 over 1000 19.1 / 12.5, 512 x 1000 over 257 12.4 / 10.2,
+// over 512 16.6 / 12.6. A wave's serial run of K, and the operands' traffic (each 32 x 32 tile reads its
+// rows and columns again) bound it: 128 x 128 over 2048 14.4 / 18.1 (split K), 1000 x 1000 over 512 17.2 /
+// 21.9. The lines leave out sizes that would still gain, by layout: up to 256 tiles K to about 1500 (128 x
+// 128 over 1280 16.3 / 13.1, over 1536 15.6 / 15.1), up to 512 tiles K to about 1000 (512 x 1000 over 640
+// 19.2 / 16.7 and, B transposed, 20.9 / 15.3; over 1024 22.3 / 21.2 and 23.4 / 19.5).
 bool gemm_takes_small(int M, int N, int K) {
     const std::int64_t tiles = static_cast<std::int64_t>(blocks_for(M, SMALL_TILE)) * blocks_for(N, SMALL_TILE);
     return M > 0 && N > 0 && K > 0 && K <= (tiles <= 256 ? 1024 : 512) && tiles <= 512;
