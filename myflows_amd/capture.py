@@ -113,7 +113,8 @@ class RecordedStep(_ReplayedStep):
     ``warmup`` eager passes run first, so that plans, weight orders and workspaces exist; then one
     more eager pass runs while the library records it (mfh_program_begin / mfh_program_end), with
     every tensor it allocates in a private memory pool: the blocks of the pass's temporaries stay
-    reserved for the replays, which write them in the recorded order. Every GPU write of the pass
+    reserved for the replays, which write them in the recorded order; the stream workspaces it uses
+    are held by the step. Every GPU write of the pass
     is a library launch (the backward's seed too), so the program is the whole pass. The same rules
     as for ``CapturedStep`` hold: fixed shapes and leaf flags, inputs refreshed in place, outputs and
     gradients overwritten by each replay, the optimiser update eager."""
@@ -127,6 +128,8 @@ class RecordedStep(_ReplayedStep):
             graph.backward()
         self.pool = torch.cuda.MemPool()
         self.program = None
+        # The launches' stream workspaces are older than the pool (the warm-up made them) or in it.
+        self._workspaces = native.stream_workspaces()
         with torch.cuda.use_mem_pool(self.pool):
             native.program_begin()
             try:

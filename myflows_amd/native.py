@@ -602,6 +602,12 @@ def stream_workspace(count, dtype=torch.float32):
     return held
 
 
+def stream_workspaces():
+    """The blocks that stream_workspace hands out now. What keeps their addresses (a recorded program)
+    keeps this list too: a larger request would otherwise give them back to the allocator."""
+    return list(_STREAM_WORKSPACES.values())
+
+
 def _holds_pending_split(block):
     return any(entry[1] is block for entry in _PENDING_SPLITS.values())
 

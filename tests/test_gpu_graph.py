@@ -325,6 +325,24 @@ def _recorded_against_eager(batch, base_width=16, shape=(48, 64), overlap=True, 
     step.close()
 
 
+def test_recorded_step_keeps_the_workspaces_its_program_writes():
+    """A later call that needs a larger stream workspace replaces the one the recorded launches use: the
+    step holds the old block, so a replay writes no tensor allocated since."""
+    recorded, _, _, _ = _resnet_step(2, seed=1)
+    step = mf.RecordedStep(recorded, warmup=1)
+    held = {(block.data_ptr(), block.dtype) for block in step._workspaces}
+    sizes = [(block.numel(), block.dtype) for block in native.stream_workspaces()]
+    assert sizes and {(block.data_ptr(), block.dtype) for block in native.stream_workspaces()} <= held
+    for numel, dtype in sizes:
+        native.stream_workspace(numel + 4096, dtype)
+    later = [torch.full((numel,), 7.0, dtype=dtype, device="cuda") for numel, dtype in sizes]
+    torch.cuda.synchronize()
+    step.one_step()
+    torch.cuda.synchronize()
+    assert all(bool((tensor == 7.0).all()) for tensor in later)
+    step.close()
+
+
 @pytest.mark.parametrize("overlap", (True, False), ids=("two-streams", "one-stream"))
 def test_recorded_step_replays_the_eager_step_bit_for_bit(overlap):
     """RecordedStep (the library's launches and stream orderings of one forward and backward pass,
